@@ -16,6 +16,7 @@ OBJ_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT_DIR, "libmfem_hip.so")
 
 SOURCES = [
+    "k_cg_resident.hip",
     "k_element.hip",
     "k_ic.hip",
     "k_minres.hip",

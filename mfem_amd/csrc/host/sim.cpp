@@ -534,6 +534,7 @@ void PcgSolver<DIM>::force_cg_shape(int variant, int blocks) {
     throw std::invalid_argument("CG grid must be 0 or a multiple of 8 in [8, 4096]");
   cg_variant_ = variant;
   cg_blocks_ = variant < 0 ? 0 : blocks;
+  cg_forced_ = variant >= 0;
 }
 
 template <int DIM>
@@ -573,9 +574,70 @@ PcgBuffers<T> PcgSolver<DIM>::buffers(const double* b, double* x) {
   return B;
 }
 
+// A forced kernel shape and the launch profile are about the
+// one-kernel-per-iteration CG.
+template <int DIM>
+CgResidentPlan PcgSolver<DIM>::resident_plan(int value_bytes) const {
+  if (cg_forced_ || this->profile_spmv || !res_fits_) return CgResidentPlan();
+  return cg_resident_plan(this->state_->mesh_->nfree(), max_row_, value_bytes);
+}
+
+template <int DIM>
+template <typename T>
+bool PcgSolver<DIM>::run_cg_resident(const double* b, double* x, double tol, int max_iters) {
+  hipStream_t st = this->state_->ctx_->stream;
+  auto& m = *this->state_->mesh_;
+  const CgResidentPlan plan = resident_plan(sizeof(T));
+  if (plan.nwg == 0) return false;
+  res_q_.resize(9 * (size_t)m.nfree(), sizeof(T) == 4);
+  res_spill_.resize(plan.spill, sizeof(T) == 4);
+  res_parts_.resize(24 * (size_t)kCgResidentMaxWg);
+  res_flag_.resize(1);
+  CgResidentArgs<T> A;
+  A.nrows = m.nfree();
+  A.rowptr = m.d_rowptr.data();
+  A.col = m.d_col.data();
+  A.K = system_.K.template as<T>();
+  A.invdiag = system_.invdiag.template as<T>();
+  A.b = b;
+  A.x = x;
+  A.tol = tol;
+  A.max_iters = max_iters;
+  A.q = reinterpret_cast<decltype(A.q)>(res_q_.template as<T>());
+  A.parts = res_parts_.data();
+  A.spill = res_spill_.template as<T>();
+  A.stride = plan.stride;
+  A.flag = res_flag_.data();
+  A.ctrl = ctrl_.data();
+  A.mirror = pinned_->device<PcgCtrl>();
+  A.wait_ticks = (long long)(this->state_->config_->resident_wait_ms * wall_khz_);
+  volatile PcgCtrl* mirror = pinned_->as<PcgCtrl>();
+  mirror->done = 0;
+  if (!launch_cg_resident<T>(A, plan.nwg, max_row_, st)) {
+    (void)hipGetLastError();
+    res_fits_ = false;
+    return false;
+  }
+  // the workgroup that writes the mirror ends whatever the others do
+  while (!mirror->done) _mm_pause();
+  std::atomic_thread_fence(std::memory_order_acquire);
+  if (mirror->done == kCgNoFit) res_fits_ = false;
+  if (mirror->done != kCgDone) return false;
+  last_ = PcgCtrl{};
+  last_.rr = mirror->rr;
+  last_.b2 = mirror->b2;
+  last_.threshold = mirror->threshold;
+  last_.iter = mirror->iter;
+  last_.done = 1;
+  last_.max_iters = mirror->max_iters;
+  last_.stop_it = mirror->stop_it;
+  return true;
+}
+
 template <int DIM>
 template <typename T>
 int PcgSolver<DIM>::run_cg(const double* b, double* x, double tol, int max_iters) {
+  if (run_cg_resident<T>(b, x, tol, max_iters)) return last_.iter;
   hipStream_t st = this->state_->ctx_->stream;
   PcgBuffers<T> B = buffers<T>(b, x);
   // Every CG kernel that does work writes its index into mapped pinned
@@ -744,7 +806,10 @@ void PcgSolver<DIM>::solve() {
     if (f32) tune_spmv<float>();
     else tune_spmv<double>();
   }
-  if (cg_variant_ < 0) {
+  if (max_row_ == 0)
+    for (int i = 0; i < m.nfree(); ++i)
+      max_row_ = std::max(max_row_, m.rowptr_[i + 1] - m.rowptr_[i]);
+  if (cg_variant_ < 0 && resident_plan(f32 ? 4 : 8).nwg == 0) {
     if (f32) tune_cg<float>();
     else tune_cg<double>();
   }
@@ -1812,6 +1877,7 @@ void SimState<DIM>::load_params(const Json& a) {
   if (a.has("newton_tol")) config_->newton_tol = a["newton_tol"].as_number();
   if (a.has("precision"))
     config_->precision = a["precision"].as_string() == "mixed" ? Precision::MIXED : Precision::FP64;
+  if (a.has("resident_wait_ms")) config_->resident_wait_ms = a["resident_wait_ms"].as_number();
   if (a.has("pcg_poll")) config_->pcg_poll = a["pcg_poll"].as_int();
 }
 

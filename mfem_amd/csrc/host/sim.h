@@ -342,6 +342,12 @@ class PcgSolver : public LinearSolver<DIM> {
   mfemhip::PcgBuffers<T> buffers(const double* b, double* x);
   template <typename T>
   int run_cg(const double* b, double* x, double tol, int max_iters);
+  // The solve in one cooperative launch (k_cg_resident.hip); false when the
+  // system does not fit, the launch was refused or a wait inside it expired,
+  // and nothing but x has changed then.
+  template <typename T>
+  bool run_cg_resident(const double* b, double* x, double tol, int max_iters);
+  mfemhip::CgResidentPlan resident_plan(int value_bytes) const;
   template <typename T>
   void tune_spmv();
   template <typename T>
@@ -356,6 +362,9 @@ class PcgSolver : public LinearSolver<DIM> {
   int variant_ = -1;
   std::vector<double> tune_ms_;
   int cg_variant_ = -1, cg_blocks_ = 0;
+  bool cg_forced_ = false;  // shape set by force_cg_shape
+  int max_row_ = 0;         // blocks in the longest row of K
+  bool res_fits_ = true;    // false once the resident CG found that K does not fit
   std::vector<CgTrial> cg_trials_;
   SystemMatrixPD<DIM> system_;
   DeviceArray<double> x_, r64_, dx64_;
@@ -364,6 +373,10 @@ class PcgSolver : public LinearSolver<DIM> {
   DeviceArray<double> parts_;    // 2 x kCgParts x kCgMaxBlocks partial sums
   DeviceArray<unsigned long long> stamps_;  // 2 x 2 x kCgMaxBlocks clock stamps
   DeviceArray<mfemhip::PcgCtrl> ctrl_;
+  RealArray res_q_;              // resident CG: exchange words of q, 3 slots
+  DeviceArray<unsigned long long> res_parts_;  // resident CG: exchanged partial sums
+  RealArray res_spill_;          // resident CG: block values beyond registers and LDS
+  DeviceArray<int> res_flag_;    // resident CG: a workgroup gave up
   mfemhip::PcgCtrl last_{};      // control block at the end of the last CG solve
   std::unique_ptr<PinnedBuffer> pinned_;  // mapped host copy of the control block
   double wall_khz_ = 100000.0;   // device wall-clock rate

@@ -5,6 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <type_traits>
 
 namespace mfemhip {
 
@@ -205,6 +206,47 @@ void launch_pcg_init(const PcgBuffers<T>& B, double tol, int max_iters, hipStrea
 // also applies the update of iteration it-1 and tests its residual).
 template <typename T>
 void launch_pcg_iteration(const PcgBuffers<T>& B, int it, hipStream_t st);
+
+// CG with the system resident in registers, one cooperative launch per solve
+// (k_cg_resident.hip): systems whose blocks fit the chip's registers.
+template <typename T>
+struct CgResidentArgs {
+  int nrows = 0;  // block rows
+  const int* rowptr = nullptr;
+  const int* col = nullptr;
+  const T* K = nullptr;
+  const T* invdiag = nullptr;
+  const double* b = nullptr;
+  double* x = nullptr;
+  double tol = 0.0;
+  int max_iters = 0;
+  typename std::conditional<sizeof(T) == 4, unsigned, unsigned long long>::type* q = nullptr;  // 9 nrows words
+  unsigned long long* parts = nullptr;  // 24 kCgResidentMaxWg words
+  T* spill = nullptr;          // CgResidentPlan::spill values
+  int stride = 1;              // CgResidentPlan::stride
+  int lds = 0;                 // dynamic LDS of a workgroup (set by the launch)
+  int* flag = nullptr;
+  PcgCtrl* ctrl = nullptr;
+  PcgCtrl* mirror = nullptr;   // as in PcgBuffers; its done is kCgDone or kCgExpired
+  long long wait_ticks = 0;    // longest wait of a workgroup for the others (wall clock)
+};
+constexpr int kCgDone = 1;
+constexpr int kCgExpired = 2;  // a wait expired: there is no solution
+constexpr int kCgNoFit = 3;    // a workgroup's columns do not fit: there is no solution
+constexpr int kCgResidentMaxWg = 256;
+constexpr int kCgResidentSpill = 8;  // most blocks of a lane in `spill`
+// Workgroups that the resident CG takes for nrows block rows of at most
+// max_row blocks (0: the system does not fit), and the values that
+// CgResidentArgs::spill needs (0: none).
+struct CgResidentPlan {
+  int nwg = 0, stride = 1;
+  long spill = 0;
+};
+CgResidentPlan cg_resident_plan(int nrows, int max_row, int value_bytes);
+// One solve (clears the exchange buffers first). False when the launch was
+// refused.
+template <typename T>
+bool launch_cg_resident(const CgResidentArgs<T>& A, int nwg, int max_row, hipStream_t st);
 
 // Batched CG over the diagonal blocks of a block-diagonal K (independent
 // simulations): workgroups [wg0[b], wg0[b+1]) own the block rows

@@ -1,0 +1,153 @@
+"""The CG with the system resident in registers (one cooperative launch per
+solve) against the one-kernel-per-iteration CG, which set_cg_shape selects, on
+the same system: every kernel of its dispatch (row lengths up to 8, 16, 32 and
+64 blocks, passes of rows, both precisions) at sizes around the edges of the
+workgroup rule. Needs an MI355X.
+
+Bars: both run Eigen's iteration from the same data and differ in the order of
+their sums only. Converged to 1e-12 (FP64; defect-corrected to 1e-10 in mixed
+precision), dx agrees to 1e-8, about the tolerance times the condition of
+these systems; iteration counts may differ by the few steps that rounding
+moves a residual of 1e-12 |b| by (2%; in mixed precision a different
+rounding also changes where the defect-correction sweeps end, so the total is
+not compared).
+"""
+import json
+import os
+
+import numpy as np
+import pytest
+
+from mfem_amd import scenes
+
+pytestmark = pytest.mark.gpu
+GOLDEN = os.path.join(os.path.dirname(__file__), "golden")
+
+
+@pytest.fixture(scope="module")
+def native():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a visible MI355X"
+    from mfem_amd import native as N
+    N.lib()
+    return N
+
+
+def solve(native, sc, precision, shape=None):
+    g = native.Sim(sc, precision=precision)
+    if shape is not None:
+        g.set_cg_shape(shape)
+    g.update_system()
+    g.solve()
+    return g.get("dx"), int(g.get_int("pcg_iters")[0]), g
+
+
+def compare(native, sc, precision):
+    sc.itr_tol = 1e-12 if precision == "fp64" else 1e-10
+    sc.max_iters = 20000
+    a, ia, g = solve(native, sc, precision)
+    b, ib, _ = solve(native, sc, precision, 0)
+    assert np.isfinite(a).all() and np.abs(b).max() > 0
+    assert np.abs(a - b).max() / np.abs(b).max() < 1e-8
+    if precision == "fp64":
+        assert abs(ia - ib) <= max(3, 0.02 * ib), (ia, ib)
+    return g
+
+
+# 1 row per workgroup .. the last size on one XCD, the first over all of them,
+# then 1, 2, 3 and 5 (FP64) or 2, 4 and 6 (mixed) passes of rows
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [(1, 1, 1), (2, 1, 2), (7, 3, 3), (32, 7, 7), (33, 7, 7), (41, 19, 20),
+                               (61, 22, 22), (60, 24, 24), (81, 25, 25), (90, 30, 30)])
+def test_beams(native, n, precision):
+    compare(native, scenes.beam_scene(*n, seed=5, mixed=n[0] % 2 == 0), precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [(9, 4), (270, 60), (270, 61), (400, 120), (700, 150), (900, 220)])
+def test_sheets(native, n, precision):
+    compare(native, scenes.rect2d_scene(*n), precision)
+
+
+def cloud_scene(points, seed, hub=0):
+    """Delaunay mesh of jittered grid points: rows of up to ~30 blocks; with
+    `hub`, points on a sphere around one vertex instead: a row of hub + 1."""
+    from scipy.spatial import Delaunay
+    rng = np.random.RandomState(seed)
+    if hub:
+        k = np.arange(hub) + 0.5
+        phi, th = np.arccos(1 - 2 * k / hub), np.pi * (1 + 5 ** 0.5) * k
+        P = np.vstack([[0.01, 0.02, 0.0], np.stack([np.cos(th) * np.sin(phi),
+                                                    np.sin(th) * np.sin(phi), np.cos(phi)], 1)])
+    else:
+        P = np.stack(np.meshgrid(*[np.arange(points)] * 3, indexing="ij"), -1).reshape(-1, 3)
+        P = P + rng.uniform(-0.35, 0.35, P.shape)
+    T = Delaunay(P).simplices.astype(np.int32)
+    D = np.stack([P[T[:, j]] - P[T[:, 0]] for j in (1, 2, 3)], 1)
+    v = np.linalg.det(D)
+    T = T[np.abs(v) > 1e-3]
+    v = v[np.abs(v) > 1e-3]
+    T[v < 0] = T[v < 0][:, [0, 2, 1, 3]]
+    used = np.unique(T)
+    renum = np.full(P.shape[0], -1, dtype=np.int32)
+    renum[used] = np.arange(used.size)
+    V, T = P[used] * 0.1, renum[T]
+    mu, la = scenes.enu_to_lame(np.full(T.shape[0], 1e6), 0.45)
+    fixed = scenes.bc_fixed("hangends", V, axis=0, ratio=0.2)
+    return scenes.Scene(V=V, T=T, mu=mu, la=la, mat=np.zeros(T.shape[0], dtype=np.int32),
+                        fixed=fixed, mixed=False)
+
+
+# rows longer than 16 (any Delaunay mesh), than 32 (a hub of 50) and than 64
+# (no kernel: the iteration falls back); 16^3 points pass 16 rows per workgroup
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("points,hub", [(6, 0), (16, 0), (27, 0), (0, 50), (0, 90)])
+def test_long_rows(native, points, hub, precision):
+    sc = cloud_scene(points, 3, hub)
+    g = compare(native, sc, precision)
+    rows = np.diff(g.get_int("bsr_rowptr"))
+    assert rows.max() > (hub * 0.6 if hub else 16)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_matches_the_oracle(native, oracle, precision):
+    sc = scenes.beam_scene(8, 3, 3, seed=7, mixed=True, E_range=(1e5, 1e6), itr_tol=1e-12,
+                           max_iters=20000)
+    o = oracle.Sim(sc)
+    o.update_system()
+    o.solve()
+    dx, it, _ = solve(native, sc, precision)
+    ref = o.get("dx")
+    # mixed: K itself is stored in FP32 (2^-24 = 6e-8 an entry), and a solve
+    # amplifies that by at most the scaled condition, about 1e2 here
+    bar = 1e-9 if precision == "fp64" else 1e2 * 2.0 ** -24
+    assert np.abs(dx - ref).max() / np.abs(ref).max() < bar
+
+
+def test_stopping_rule(native):
+    """The iteration cap, and zero iterations for |b|^2 below tol^2 |b|^2."""
+    for kw, want in ((dict(max_iters=3), 3), (dict(max_iters=1), 1), (dict(itr_tol=2.0), 0)):
+        sc = scenes.beam_scene(8, 3, 3, seed=7, mixed=True, **kw)
+        a, ia, g = solve(native, sc, "fp64")
+        b, ib, _ = solve(native, sc, "fp64", 0)
+        assert ia == ib == want
+        assert np.allclose(a, b, rtol=0, atol=1e-12 * max(1.0, np.abs(b).max()))
+
+
+def test_expired_wait_falls_back(native, tmp_path):
+    """With no time to wait for each other the workgroups leave, and the solve
+    runs as one kernel per iteration: the same step."""
+    scene = json.load(open(os.path.join(GOLDEN, "beam_scene.json")))
+    scene["objects"][0]["path"] = os.path.join(GOLDEN, scene["objects"][0]["path"])
+    scene["linear_solver"] = "eigen-pcg-diag"
+    out = []
+    for wait in (2000, 0):
+        scene["resident_wait_ms"] = wait
+        path = tmp_path / f"scene{wait}.json"
+        path.write_text(json.dumps(scene))
+        g = native.Sim(json_path=str(path))
+        for _ in range(2):
+            g.step()
+        out.append((g.positions(), g.stats()["newton_iters"]))
+    assert out[0][1] == out[1][1]
+    assert np.abs(out[0][0] - out[1][0]).max() < 1e-8
