@@ -4,7 +4,8 @@
 // ConjugateGradient<SpMat, Lower|Upper> with its default DiagonalPreconditioner,
 // reference src/linear_solvers/eigen_iterative_solver.h:14-29, configured by
 // src/factories/linear_solver_factory.cpp:75-85). The iteration itself is the
-// library's one-kernel-per-iteration CG (k_solver.hip), in FP64.
+// library's resident CG (k_cg_resident.hip) where the system fits the chip, else
+// its one-kernel-per-iteration CG (k_solver.hip), in FP64.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,24 +24,26 @@ namespace {
 
 constexpr int kCheckBS = 256;
 
-__global__ void k_zero_flag(int* flag) { *flag = 0; }
+__global__ void k_zero_flag(int* flag) { flag[0] = flag[1] = 0; }
 
 // Pattern check and Eigen's DiagonalPreconditioner::factorize (1 / a_jj, or 1
 // where the diagonal entry is zero or absent; the first diagonal block of a
-// row counts). One block row per lane. flag bit 0: rowptr[0] != 0, a row
+// row counts). One block row per lane. flag[0] bit 0: rowptr[0] != 0, a row
 // pointer out of order or past nnzb; bit 1: a block column outside [0, nb).
+// flag[1]: blocks in the longest row.
 __global__ __launch_bounds__(kCheckBS) void k_bsr_check_invdiag(
     int nb, int nnzb, const int* __restrict__ rowptr, const int* __restrict__ col,
     const double* __restrict__ K, double* __restrict__ invdiag, int* flag) {
   const int i = blockIdx.x * kCheckBS + threadIdx.x;
-  if (i >= nb) return;
-  const int p0 = rowptr[i], p1 = rowptr[i + 1];
+  const bool on = i < nb;
+  const int p0 = on ? rowptr[i] : 0, p1 = on ? rowptr[i + 1] : 0;
   double d[3] = {1.0, 1.0, 1.0};
-  int bad = (i == 0 && p0 != 0) ? 1 : 0;
+  int bad = (i == 0 && p0 != 0) ? 1 : 0, len = 0;
   if (p0 < 0 || p1 < p0 || p1 > nnzb) {
     bad |= 1;
   } else {
     bool found = false;
+    len = p1 - p0;
     for (int b = p0; b < p1; ++b) {
       const int c = col[b];
       if (c < 0 || c >= nb) {
@@ -55,9 +58,14 @@ __global__ __launch_bounds__(kCheckBS) void k_bsr_check_invdiag(
       }
     }
   }
+  if (on) {
 #pragma unroll
-  for (int r = 0; r < 3; ++r) invdiag[3L * i + r] = d[r];
+    for (int r = 0; r < 3; ++r) invdiag[3L * i + r] = d[r];
+  }
   if (bad) atomicOr(flag, bad);
+  // one atomic per wave: the longest row of the active lanes
+  for (int off = 32; off > 0; off >>= 1) len = max(len, __shfl_xor(len, off));
+  if ((threadIdx.x & 63) == 0) atomicMax(flag + 1, len);
 }
 
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -74,7 +82,7 @@ struct PcgWorkLayout {
     ctrl = o;
     o += align256(sizeof(PcgCtrl));
     flag = o;
-    o += align256(sizeof(int));
+    o += align256(3 * sizeof(int));
     parts = o;
     o += align256(sizeof(double) * 2 * kCgParts * (size_t)kCgMaxBlocks);
     invdiag = o;
@@ -113,12 +121,49 @@ void pcg_bsr3_run(char* work, int nb, int nnzb, const int* rowptr, const int* co
   hipLaunchKernelGGL(k_bsr_check_invdiag, dim3((nb + kCheckBS - 1) / kCheckBS), dim3(kCheckBS), 0,
                      st, nb, nnzb, rowptr, col, vals, invdiag, flag);
   MFEM_HIP_CHECK(hipGetLastError());
-  int hflag = 0;
-  MFEM_HIP_CHECK(hipMemcpyAsync(&hflag, flag, sizeof(int), hipMemcpyDeviceToHost, st));
+  int hflag[2] = {0, 0};
+  MFEM_HIP_CHECK(hipMemcpyAsync(hflag, flag, sizeof(hflag), hipMemcpyDeviceToHost, st));
   MFEM_HIP_CHECK(hipStreamSynchronize(st));
-  if (hflag & 1) throw std::invalid_argument("malformed block row pointer (rowptr)");
-  if (hflag & 2) throw std::invalid_argument("block column index out of range");
+  if (hflag[0] & 1) throw std::invalid_argument("malformed block row pointer (rowptr)");
+  if (hflag[0] & 2) throw std::invalid_argument("block column index out of range");
 
+  PcgCtrl h{};
+  auto finish = [&] {
+    if (iterations) *iterations = h.iter;
+    if (rel_residual) *rel_residual = h.b2 > 0 ? std::sqrt(h.rr / h.b2) : 0.0;
+  };
+  // a system that fits the chip: every iteration in one launch, with its
+  // exchange buffers in the work arrays of the path below
+  const CgResidentPlan plan = cg_resident_plan(nb, hflag[1], sizeof(double));
+  if (plan.nwg > 0 && plan.spill == 0) {
+    CgResidentArgs<double> A;
+    A.nrows = nb;
+    A.rowptr = rowptr;
+    A.col = col;
+    A.K = vals;
+    A.invdiag = invdiag;
+    A.b = b;
+    A.x = x;
+    A.tol = tol;
+    A.max_iters = max_iters;
+    A.q = reinterpret_cast<unsigned long long*>(work + L.state0);
+    A.parts = reinterpret_cast<unsigned long long*>(work + L.parts);
+    A.stride = plan.stride;
+    A.flag = flag + 2;
+    A.ctrl = reinterpret_cast<PcgCtrl*>(work + L.ctrl);
+    int dev = 0, khz = 0;
+    MFEM_HIP_CHECK(hipGetDevice(&dev));
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)
+      khz = 100000;
+    A.wait_ticks = 2000LL * khz;
+    if (launch_cg_resident(A, plan.nwg, hflag[1], st)) {
+      MFEM_HIP_CHECK(hipMemcpyAsync(&h, A.ctrl, sizeof(PcgCtrl), hipMemcpyDeviceToHost, st));
+      MFEM_HIP_CHECK(hipStreamSynchronize(st));
+      if (h.done == kCgDone) return finish();
+    } else {
+      (void)hipGetLastError();
+    }
+  }
   PcgBuffers<double> B;
   B.n = n;
   B.rowptr = rowptr;
@@ -139,7 +184,6 @@ void pcg_bsr3_run(char* work, int nb, int nnzb, const int* rowptr, const int* co
   // 16 launches, and launches queued after the stop exit at once
   const long limit = (long)max_iters + 2;
   long launched = 0;
-  PcgCtrl h{};
   while (true) {
     const long chunk = std::min<long>(16, limit - launched);
     for (long j = 0; j < chunk; ++j) launch_pcg_iteration(B, (int)(launched + j), st);
@@ -150,8 +194,7 @@ void pcg_bsr3_run(char* work, int nb, int nnzb, const int* rowptr, const int* co
     if (h.done) break;
     if (launched >= limit) throw std::runtime_error("CG control block did not terminate");
   }
-  if (iterations) *iterations = h.iter;
-  if (rel_residual) *rel_residual = h.b2 > 0 ? std::sqrt(h.rr / h.b2) : 0.0;
+  finish();
 }
 
 }  // namespace mfemhip
@@ -194,6 +237,7 @@ constexpr size_t kNoAllocBytes =
     sizeof(double) * 9 * (size_t)kNoAllocRows + sizeof(double) * 2 * kCgParts * kCgMaxBlocks +
     4 * 256;
 static_assert(kNoAllocBytes % sizeof(double) == 0, "scratch size");
+static_assert(24 * kCgResidentMaxWg <= 2 * kCgParts * kCgMaxBlocks, "resident CG's sums fit");
 
 static __device__ __align__(256) double scratch[kNoAllocBytes / sizeof(double)];
 

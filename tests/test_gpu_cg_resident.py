@@ -151,3 +151,54 @@ def test_expired_wait_falls_back(native, tmp_path):
         out.append((g.positions(), g.stats()["newton_iters"]))
     assert out[0][1] == out[1][1]
     assert np.abs(out[0][0] - out[1][0]).max() < 1e-8
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (4, 3, 2), (9, 7, 5), (20, 16, 13), (40, 40, 32)])
+def test_caller_matrices(native, n):
+    """mfem_pcg_bsr3 with the forms it accepts: columns in any order, a column
+    twice in a row, rows without a diagonal block (a zero right-hand side
+    there). The last size is past the resident CG's, and goes the other way.
+    Against K x = b itself: the residual is what the call says it is, in the
+    2-norm to the rounding of K x (1e-14 of |K||x| per product), and below
+    tol."""
+    import torch
+    rng = np.random.RandomState(n[0])
+    ids = np.arange(np.prod(n)).reshape(n)
+    rows, cols, vals = [], [], []
+    diag = np.tile(1e-2 * np.eye(3), (ids.size, 1, 1))
+    for ax in range(3):
+        i = ids.take(range(n[ax] - 1), axis=ax).ravel()
+        j = ids.take(range(1, n[ax]), axis=ax).ravel()
+        A = rng.randn(i.size, 3, 3)
+        W = A @ A.transpose(0, 2, 1) + 0.3 * np.eye(3)
+        np.add.at(diag, i, W)
+        np.add.at(diag, j, W)
+        rows += [i, j]
+        cols += [j, i]
+        vals += [-W, -W]
+    bare = ids.ravel()[::17][1:]  # rows and columns without any block
+    keep = np.ones(ids.size, dtype=bool)
+    keep[bare] = False
+    part = rng.rand(ids.size, 1, 1)  # the diagonal block in two pieces
+    rows += [ids.ravel()[keep]] * 2
+    cols += [ids.ravel()[keep]] * 2
+    vals += [(part * diag)[keep], ((1 - part) * diag)[keep]]
+    rows, cols, vals = np.concatenate(rows), np.concatenate(cols), np.concatenate(vals)
+    on = keep[rows] & keep[cols]
+    rows, cols, vals = rows[on], cols[on], vals[on]
+    order = np.lexsort((rng.rand(rows.size), rows))
+    rows, cols, vals = rows[order], cols[order], vals[order]
+    rowptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=ids.size))]).astype(np.int32)
+    b = rng.randn(ids.size, 3)
+    b[bare] = 0.0
+    dev = [torch.as_tensor(np.ascontiguousarray(a), device="cuda")
+           for a in (rowptr, cols.astype(np.int32), vals.reshape(-1), b.reshape(-1))]
+    tol = 1e-9
+    x, it, rr = native.pcg_bsr3(*dev, tol, 20000)
+    x = x.cpu().numpy().reshape(-1, 3)
+    r = b.copy()
+    np.subtract.at(r, rows, (vals @ x[cols][:, :, None])[:, :, 0])
+    true = np.linalg.norm(r) / np.linalg.norm(b)
+    assert np.isfinite(x).all() and it < 20000 and rr < tol
+    assert abs(true - rr) < 1e-14 * np.abs(vals).sum((1, 2)).max() * np.linalg.norm(x) / np.linalg.norm(b) * max(it, 1)
+    assert not np.any(x[bare])
