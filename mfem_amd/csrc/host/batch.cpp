@@ -99,6 +99,10 @@ BatchSim::BatchSim(const std::vector<SceneArrays>& sims, std::shared_ptr<SimConf
   d_on_.resize(nsim_);
   e_tet_.resize((size_t)S.mesh_->nT());
   scratch_.resize(256);
+  int dev = 0, khz = 0;
+  MFEM_HIP_CHECK(hipGetDevice(&dev));
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0)
+    wall_khz_ = khz;
   res_.assign((size_t)RES_ROWS * nsim_, 0.0);
   stats_.resize(nsim_);
   MFEM_HIP_CHECK(hipStreamSynchronize(st));
@@ -189,8 +193,12 @@ void BatchSim::update_and_assemble(double dt) {
 std::vector<double> BatchSim::positions(int sim) const {
   if (sim < 0 || sim >= nsim_) throw std::runtime_error("batch: simulation index out of range");
   auto& S = *state_;
-  const auto x = S.x_->value().to_host(S.ctx_->stream);
-  return std::vector<double>(x.begin() + 3 * (size_t)v0_[sim], x.begin() + 3 * (size_t)v0_[sim + 1]);
+  std::vector<double> x(3 * (size_t)(v0_[sim + 1] - v0_[sim]));
+  MFEM_HIP_CHECK(hipMemcpyAsync(x.data(), S.x_->value().data() + 3 * (size_t)v0_[sim],
+                                x.size() * sizeof(double), hipMemcpyDeviceToHost,
+                                S.ctx_->stream));
+  MFEM_HIP_CHECK(hipStreamSynchronize(S.ctx_->stream));
+  return x;
 }
 
 template <typename T>
@@ -210,6 +218,7 @@ void BatchSim::force_cg_shape(int variant, int rows_per_wg) {
   if (variant >= 0 && rows_per_wg <= 0) throw std::invalid_argument("rows per workgroup must be > 0");
   variant_ = variant;
   rows_per_wg_ = variant < 0 ? 0 : rows_per_wg;
+  cg_forced_ = variant >= 0;
   if (variant >= 0) layout_workgroups(rows_per_wg_);
 }
 
@@ -260,6 +269,130 @@ BatchCgBuffers<T> BatchSim::buffers(const double* b, double* x) {
   return B;
 }
 
+int BatchSim::resident_passes(int value_bytes) {
+  if (cg_forced_ || !res_fits_) return 0;
+  if (res_passes_ < 0) {
+    const auto& rp = state_->mesh_->rowptr_;
+    for (size_t i = 0; i + 1 < rp.size(); ++i) max_row_ = std::max(max_row_, rp[i + 1] - rp[i]);
+    res_passes_ = cg_resident_batch_passes(f0_.data(), nsim_, max_row_, value_bytes,
+                                           &res_spill_n_);
+  }
+  return res_passes_;
+}
+
+template <typename T>
+bool BatchSim::run_cg_resident(const double* b, double* x, const std::vector<double>& tol,
+                               const std::vector<int>& budget, const std::vector<int>& on,
+                               std::vector<int>& iters) {
+  const int passes = resident_passes(sizeof(T));
+  if (passes == 0) return false;
+  auto& S = *state_;
+  auto& m = *S.mesh_;
+  hipStream_t st = S.ctx_->stream;
+  // Systems to teams, longest first to the team that is free first: the teams
+  // of a whole XCD, then the small ones inside each XCD behind them. The cost
+  // is the last solve's iterations (which team solves a system changes no bit
+  // of it).
+  constexpr int kXcds = 8, kSub = kCgTeamLarge / kCgTeamSmall;
+  if ((int)res_cost_.size() != nsim_) res_cost_.assign(nsim_, 0.0);
+  auto cost = [&](int k) {
+    const int rows = f0_[k + 1] - f0_[k];
+    const double it = res_cost_[k] > 0 ? res_cost_[k] : 50.0 + std::cbrt((double)rows) * 5.0;
+    return (std::min<double>(it, budget[k]) + 4.0) *
+           (3.0 + rows / (64.0 * cg_team_of(rows, nsim_)));
+  };
+  std::vector<int> order;
+  for (int k = 0; k < nsim_; ++k)
+    if (on[k] && f0_[k + 1] > f0_[k]) order.push_back(k);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return cost(a) > cost(c); });
+  std::vector<std::vector<int>> large(kXcds), small(kXcds * kSub);
+  std::vector<double> load(kXcds * kSub, 0.0);
+  for (int pass = 0; pass < 2; ++pass)
+    for (int k : order) {
+      const bool big = cg_team_of(f0_[k + 1] - f0_[k], nsim_) == kCgTeamLarge;
+      if (big != (pass == 0)) continue;
+      int t = 0;
+      if (big) {
+        for (int q = 1; q < kXcds; ++q)
+          if (load[q * kSub] < load[t * kSub]) t = q;
+        large[t].push_back(k);
+        for (int q = 0; q < kSub; ++q) load[t * kSub + q] += cost(k);
+      } else {
+        t = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        small[t].push_back(k);
+        load[t] += cost(k);
+      }
+    }
+  if (!res_stage_)
+    res_stage_ = std::make_unique<PinnedBuffer>(sizeof(CgResidentSys) * nsim_ + 64 * sizeof(int));
+  auto* hs = res_stage_->as<CgResidentSys>();
+  int* ht = reinterpret_cast<int*>(hs + nsim_);
+  int n = 0, t = 0;
+  for (const auto* lists : {&large, &small}) {
+    for (const auto& l : *lists) {
+      ht[t++] = n;
+      for (int k : l) hs[n++] = CgResidentSys{f0_[k], f0_[k + 1], budget[k], k, tol[k]};
+    }
+    ht[t++] = n;
+  }
+  res_sys_.resize(nsim_);
+  res_team_.resize(64);
+  res_q_.resize(9 * (size_t)m.nfree(), sizeof(T) == 4);
+  res_parts_.resize(48 * (size_t)kCgResidentMaxWg);
+  res_spill_.resize(res_spill_n_, sizeof(T) == 4);
+  res_flag_.resize(1);
+  MFEM_HIP_CHECK(hipMemcpyAsync(res_sys_.data(), hs, sizeof(CgResidentSys) * n,
+                                hipMemcpyHostToDevice, st));
+  MFEM_HIP_CHECK(hipMemcpyAsync(res_team_.data(), ht, sizeof(int) * t, hipMemcpyHostToDevice, st));
+  CgResidentArgs<T> A;
+  A.nrows = m.nfree();
+  A.rowptr = m.d_rowptr.data();
+  A.col = m.d_col.data();
+  A.K = system_.K.template as<T>();
+  A.invdiag = system_.invdiag.template as<T>();
+  A.b = b;
+  A.x = x;
+  A.q = reinterpret_cast<decltype(A.q)>(res_q_.template as<T>());
+  A.parts = res_parts_.data();
+  A.spill = res_spill_.template as<T>();
+  A.flag = res_flag_.data();
+  A.ctrl = ctrls_.data();
+  A.mirror = pinned_ctrl_->device<PcgCtrl>();
+  A.sys = res_sys_.data();
+  A.team = res_team_.data();
+  A.wait_ticks = (long long)(S.config_->resident_wait_ms * wall_khz_);
+  volatile PcgCtrl* mirror = pinned_ctrl_->as<PcgCtrl>();
+  for (int k = 0; k < nsim_; ++k) mirror[k].done = 0;
+  const bool launched = launch_cg_resident_batch<T>(A, passes, max_row_, st);
+  if (!launched) (void)hipGetLastError();
+  MFEM_HIP_CHECK(hipStreamSynchronize(st));
+  std::atomic_thread_fence(std::memory_order_acquire);
+  bool ok = launched;
+  for (int k : order) {
+    ok = ok && mirror[k].done == kCgDone;
+    if (mirror[k].done == kCgNoFit) res_fits_ = false;
+  }
+  if (!launched) res_fits_ = false;
+  if (!ok) return false;
+  ++subs_cg_;
+  iters.assign(nsim_, 0);
+  for (int k = 0; k < nsim_; ++k) {
+    PcgCtrl& c = ctrl_host_[k];
+    c = PcgCtrl{};
+    c.done = 1;
+    c.max_iters = budget[k];
+    if (!on[k]) continue;
+    c.rr = mirror[k].rr;
+    c.b2 = mirror[k].b2;
+    c.threshold = mirror[k].threshold;
+    c.iter = mirror[k].iter;
+    c.stop_it = mirror[k].stop_it;
+    iters[k] = c.iter;
+    res_cost_[k] = std::max(1, c.iter);
+  }
+  return true;
+}
+
 // One batched CG solve (Eigen semantics per system, reference
 // eigen_iterative_solver.h:20-29): x = 0, per-system tolerance and
 // iteration budget; systems with on[b] = 0 are skipped (x stays 0).
@@ -267,6 +400,8 @@ template <typename T>
 void BatchSim::run_cg(const double* b, double* x, const std::vector<double>& tol,
                       const std::vector<int>& budget, const std::vector<int>& on,
                       std::vector<int>& iters) {
+  if (run_cg_resident<T>(b, x, tol, budget, on, iters)) return;
+  if (nwg_ == 0) prepare_lockstep<T>();
   auto& S = *state_;
   hipStream_t st = S.ctx_->stream;
   const BatchCgBuffers<T> B = buffers<T>(b, x);
@@ -453,6 +588,17 @@ void BatchSim::tune() {
   layout_workgroups(rows_per_wg_);
 }
 
+// The workgroup layout of the lockstep CG.
+template <typename T>
+void BatchSim::prepare_lockstep() {
+  auto& S = *state_;
+  const size_t n = 3 * (size_t)S.mesh_->nfree();
+  state0_.resize(4 * n, sizeof(T) == 4);
+  state1_.resize(4 * n, sizeof(T) == 4);
+  if (variant_ < 0) tune<T>();
+  else if (nwg_ == 0) layout_workgroups(rows_per_wg_);
+}
+
 // Linear solve of every simulation that is on (PcgSolver::solve per system:
 // FP64 CG, or FP32 CG sweeps in FP64 defect correction); dx in x_->delta()
 // and the local solve for (lambda, ds) afterwards.
@@ -464,13 +610,9 @@ void BatchSim::solve(const std::vector<int>& on) {
   const int n = 3 * m.nfree();
   const bool f32 = S.ctx_->fp32();
   x_.resize(n);
-  state0_.resize(4 * (size_t)n, f32);
-  state1_.resize(4 * (size_t)n, f32);
-  if (variant_ < 0) {
-    if (f32) tune<float>();
-    else tune<double>();
-  } else if (nwg_ == 0) {
-    layout_workgroups(rows_per_wg_);
+  if (resident_passes(f32 ? 4 : 8) == 0) {
+    if (f32) prepare_lockstep<float>();
+    else prepare_lockstep<double>();
   }
   solve_iters_.assign(nsim_, 0);
   solve_sweeps_.assign(nsim_, 0);

@@ -75,6 +75,15 @@ class BatchSim {
   void run_cg(const double* b, double* x, const std::vector<double>& tol,
               const std::vector<int>& budget, const std::vector<int>& on,
               std::vector<int>& iters);
+  // The same solve in one cooperative launch (k_cg_resident.hip); false when a
+  // system does not fit its team, the launch was refused or a wait expired.
+  template <typename T>
+  bool run_cg_resident(const double* b, double* x, const std::vector<double>& tol,
+                       const std::vector<int>& budget, const std::vector<int>& on,
+                       std::vector<int>& iters);
+  int resident_passes(int value_bytes);
+  template <typename T>
+  void prepare_lockstep();
   template <typename T>
   void tune();
   void layout_workgroups(int rows_per_wg);
@@ -103,6 +112,17 @@ class BatchSim {
   DeviceArray<mfemhip::PcgCtrl> ctrls_;
   DeviceArray<int> d_budget_, d_on_;
   std::vector<mfemhip::PcgCtrl> ctrl_host_;
+  // resident CG: see CgResidentArgs
+  bool cg_forced_ = false, res_fits_ = true;
+  int res_passes_ = -1, max_row_ = 0;
+  long res_spill_n_ = 0;
+  RealArray res_q_, res_spill_;
+  DeviceArray<unsigned long long> res_parts_;
+  DeviceArray<int> res_flag_, res_team_;
+  DeviceArray<mfemhip::CgResidentSys> res_sys_;
+  std::unique_ptr<PinnedBuffer> res_stage_;  // source of res_sys_ and res_team_
+  double wall_khz_ = 100000.0;               // device wall-clock rate
+  std::vector<double> res_cost_;             // iterations of each system's last solve
   // mapped copy of every system's control block, then the progress word
   std::unique_ptr<PinnedBuffer> pinned_ctrl_;
   // Compacted lists of the workgroups of the systems still iterating (eager

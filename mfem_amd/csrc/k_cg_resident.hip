@@ -151,6 +151,9 @@ __device__ __forceinline__ void publish_stop(const PcgCtrl& c, PcgCtrl* ctrl, Pc
   __hip_atomic_store(&mirror->done, c.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// v, the same in every lane, as one scalar
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // Flag word of a solve: 0 while it runs, 1 after a wait expired.
 struct Waiter {
   int* flag;
@@ -210,6 +213,11 @@ struct ResidentLds {
 // that the workgroup's rows touch are numbered locally (ascending); their p
 // lives in LDS, their r and D^-1 with the thread that updates them, EPT scalar
 // columns ("entries") per thread.
+//
+// One system takes all workgroups. Of many independent ones (A.sys) each is
+// solved by a team on one XCD, 32 workgroups for the large systems (phase 0)
+// and then 8 for the small ones (phase 1); a team takes its list of systems
+// one after the other, its slots rotating on.
 template <int G, int U, int R, int NREG, int NLDS, int EPT, int BS, typename T>
 __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   using W = typename Word<T>::U;
@@ -228,29 +236,60 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   __shared__ unsigned s_scan[BS / kWave];
   __shared__ int s_dead;
   if (blockIdx.x % A.stride) return;
-  const int tid = threadIdx.x, lane = tid & (G - 1), wid = tid / kWave;
-  const int nw = gridDim.x / A.stride;
-  // workgroups go round-robin over the 8 XCDs: neighbouring rows on one XCD
-  int wg = blockIdx.x / A.stride;
-  if (A.stride == 1 && (nw & 7) == 0) wg = (blockIdx.x & 7) * (nw >> 3) + (blockIdx.x >> 3);
-  const int c0 = (int)((long long)A.nrows * wg / nw);
-  const int c1 = (int)((long long)A.nrows * (wg + 1) / nw);
   const unsigned n = 3u * (unsigned)A.nrows;
+  for (int phase = 0; phase < (A.sys ? 2 : 1); ++phase) {
+  int nw = gridDim.x / A.stride;  // workgroups of the team
+  int wg;                         // this one's number in it
+  int g0 = 0;                     // the team's first place in A.parts
+  int s0 = 0, s1 = 1;             // its systems
+  if (A.sys) {
+    nw = phase ? kCgTeamSmall : kCgTeamLarge;
+    const int g = (blockIdx.x & 7) * kCgTeamLarge + (blockIdx.x >> 3);
+    wg = g % nw;
+    g0 = g - wg;
+    const int* t = A.team + (phase ? 9 : 0) + g / nw;
+    s0 = uniform(t[0]);
+    s1 = uniform(t[1]);
+  } else {
+    // workgroups go round-robin over the 8 XCDs: neighbouring rows on one XCD
+    wg = blockIdx.x / A.stride;
+    if (A.stride == 1 && (nw & 7) == 0) wg = (blockIdx.x & 7) * (nw >> 3) + (blockIdx.x >> 3);
+  }
+  U64* const parts = A.parts + (size_t)phase * 3 * kCgResidentMaxWg * 8;
+  int slot = 0, prev = 2, prev2 = 1;  // iterations it, it-1 and it-2 of the team, modulo 3
+  bool used = false;                  // slot prev2 holds sums
+  for (int si = s0; si < s1; ++si) {
+  // (nothing of a lane is kept in registers from one system to the next)
+  const int tid = opaque(threadIdx.x), lane = tid & (G - 1), wid = tid / kWave;
+  CgResidentSys sys{0, A.nrows, A.max_iters, 0, A.tol};
+  if (A.sys) {
+    const CgResidentSys q = A.sys[si];
+    sys = CgResidentSys{uniform(q.row0), uniform(q.row1), uniform(q.max_iters), uniform(q.id),
+                        q.tol};
+  }
+  PcgCtrl* const ctrl = A.ctrl + sys.id;
+  PcgCtrl* const mirror = A.mirror ? A.mirror + sys.id : nullptr;
+  const int nrows = sys.row1 - sys.row0;
+  const int c0 = sys.row0 + (int)((long long)nrows * wg / nw);
+  const int c1 = sys.row0 + (int)((long long)nrows * (wg + 1) / nw);
+  const int rows = c1 - c0;
+  __syncthreads();  // the LDS of the previous system
   if (tid == 0) s_dead = 0;
 
   // local numbering of the columns: a bit per block row, ranks by popcount
   unsigned* const list = reinterpret_cast<unsigned*>(dyn + L::list);
-  const int nword = (A.nrows + 31) / 32;
+  const int nword = (nrows + 31) / 32;
   unsigned* const bits = reinterpret_cast<unsigned*>(dyn + L::start);
   unsigned* const pre = bits + nword;
   for (int i = tid; i < nword; i += BS) bits[i] = 0;
   __syncthreads();
   const int b0 = A.rowptr[c0], b1 = A.rowptr[c1];
   for (int q = b0 + tid; q < b1; q += BS) {
-    const unsigned j = A.col[q];
+    const unsigned j = A.col[q] - sys.row0;
     atomicOr(&bits[j >> 5], 1u << (j & 31));
   }
-  for (int i = c0 + tid; i < c1; i += BS) atomicOr(&bits[i >> 5], 1u << (i & 31));
+  for (int i = c0 - sys.row0 + tid; i < c1 - sys.row0; i += BS)
+    atomicOr(&bits[i >> 5], 1u << (i & 31));
   __syncthreads();
   const int per = (nword + BS - 1) / BS;
   const int i0 = min(nword, tid * per), i1 = min(nword, i0 + per);
@@ -260,16 +299,17 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   for (int i = i0; i < i1; ++i) {
     pre[i] = at;
     for (unsigned m = bits[i]; m; m &= m - 1) {
-      if (at < (unsigned)L::kList) list[at] = 32u * i + (__ffs(m) - 1);
+      if (at < (unsigned)L::kList) list[at] = sys.row0 + 32u * i + (__ffs(m) - 1);
       ++at;
     }
   }
   __syncthreads();
   auto rank = [&](unsigned j) {
+    j -= sys.row0;
     return pre[j >> 5] + __popc(bits[j >> 5] & ((1u << (j & 31)) - 1u));
   };
-  const unsigned H = pre[nword - 1] + __popc(bits[nword - 1]);
-  const unsigned nent = 3 * H, own0 = 3 * rank(c0), nown = 3 * (c1 - c0);
+  const unsigned H = uniform(pre[nword - 1] + __popc(bits[nword - 1]));
+  const unsigned nent = 3 * H, own0 = 3 * uniform(rank(c0)), nown = 3 * (c1 - c0);
   // p has one more row, of zeros, for the lanes without a block
   const size_t pbytes = (size_t)(nent + 3) * sizeof(T);
   if (H > (unsigned)L::kList || L::p + pbytes > (size_t)A.lds || pbytes > 65536) {
@@ -278,7 +318,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
     if (tid == 0 && wg == 0) {
       PcgCtrl o{};
       o.done = kCgNoFit;
-      publish_stop(o, A.ctrl, A.mirror);
+      publish_stop(o, ctrl, mirror);
     }
     return;
   }
@@ -300,7 +340,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   T* const dl = reinterpret_cast<T*>(dyn + L::d);
   T* const ql = reinterpret_cast<T*>(dyn + L::q);
   T* const pl = reinterpret_cast<T*>(dyn + L::p);
-  T* const vs = A.spill + (size_t)wg * NSTR * 9 * BS;  // [NSTR][9][BS]
+  T* const vs = A.spill + (size_t)(g0 + wg) * NSTR * 9 * BS;  // [NSTR][9][BS]
   T V[NREG][9];
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
@@ -338,7 +378,6 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   }
   for (unsigned e = EPT * BS + tid; e < nent + 3; e += BS) pl[e] = (T)0;  // the zero row
   double threshold = 0.0, b2 = 0.0, alpha = 0.0, beta = 0.0;
-  int slot = 0, prev = 2, prev2 = 1;  // it, it-1 and it-2 modulo 3
   int done = kCgExpired;
   for (int it = 0;; ++it) {
     Waiter wait{A.flag, A.wait_ticks};
@@ -359,7 +398,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
       }
       // sum `wid` of iteration it-1 over the workgroups
       if (wid < kCgParts || (wid == kCgParts && it == 1)) {
-        const U64* src = A.parts + (size_t)prev * kCgResidentMaxWg * 8 + wid;
+        const U64* src = parts + ((size_t)prev * kCgResidentMaxWg + g0) * 8 + wid;
         U64 s[kPolls];
 #pragma unroll
         for (int h = 0; h < kPolls; ++h) {
@@ -382,14 +421,17 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
       if (dead) s_dead = 1;
       __syncthreads();
       if (s_dead) break;
+      // slot it-2 has been read everywhere: empty it for it+1
+      if (used && tid < NP)
+        word_store(parts + ((size_t)prev2 * kCgResidentMaxWg + g0 + wg) * 8 + tid, kEmpty64);
       const double pq = s_tot[0], zq = s_tot[1], qdq = s_tot[2], rr = s_tot[3], rz = s_tot[4];
       if (it == 1) {
         b2 = s_tot[kCgParts];
-        threshold = fmax(A.tol * A.tol * b2, DBL_MIN);
+        threshold = fmax(sys.tol * sys.tol * b2, DBL_MIN);
       }
       const int jt = it - 1;  // iteration of the sums
       const bool converged = rr < threshold || b2 == 0.0;
-      if (converged || jt >= A.max_iters) {
+      if (converged || jt >= sys.max_iters) {
         if (wg == 0 && tid == 0) {
           PcgCtrl o{};
           o.rr = rr;
@@ -397,10 +439,10 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
           o.threshold = threshold;
           o.iter = converged ? (jt > 0 ? jt - 1 : 0) : jt;
           o.done = kCgDone;
-          o.max_iters = A.max_iters;
+          o.max_iters = sys.max_iters;
           o.stop_it = it;
           o.started = it;
-          publish_stop(o, A.ctrl, A.mirror);
+          publish_stop(o, ctrl, mirror);
         }
         done = kCgDone;
         break;
@@ -415,9 +457,6 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
 #pragma unroll
     for (int k = 0; k < NP; ++k) acc[k] = 0.0;
     acc[kCgParts] = bb;
-    // slot it-2 has been read everywhere: empty it for it+1
-    if (it > 1 && tid < NP)
-      word_store(A.parts + ((size_t)prev2 * kCgResidentMaxWg + wg) * 8 + tid, kEmpty64);
     W* old = A.q + (size_t)prev2 * n;
     {
       const unsigned t = (kLean ? opaque(tid) : (unsigned)tid);
@@ -455,6 +494,8 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
     T q[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
+      q[j] = (T)0;
+      if (R > 1 && j * (BS / G) >= rows) continue;  // no rows in this pass
       // one pass's loads at a time where registers are short
       if constexpr (NSTR > 0 || NLDS > 0) asm volatile("" ::: "memory");
       T y0 = 0, y1 = 0, y2 = 0;
@@ -519,29 +560,36 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
       }
       t = wave_sum_63(t);
       if ((tid & (kWave - 1)) == kWave - 1)
-        word_store(A.parts + ((size_t)slot * kCgResidentMaxWg + wg) * 8 + wid,
+        word_store(parts + ((size_t)slot * kCgResidentMaxWg + g0 + wg) * 8 + wid,
                    __builtin_bit_cast(U64, t));
     }
+    used = used || it > 0 || si > s0;
     prev2 = prev;
     prev = slot;
     slot = slot == 2 ? 0 : slot + 1;
   }
-  if (done != kCgDone && wg == 0 && tid == 0) {  // x is not a solution
-    PcgCtrl o{};
-    o.done = word_load(A.flag) == kCgNoFit ? kCgNoFit : kCgExpired;
-    publish_stop(o, A.ctrl, A.mirror);
+  if (done != kCgDone) {  // x is not a solution
+    if (wg == 0 && tid == 0) {
+      PcgCtrl o{};
+      o.done = word_load(A.flag) == kCgNoFit ? kCgNoFit : kCgExpired;
+      publish_stop(o, ctrl, mirror);
+    }
+    return;
   }
   // the solution (the iterate of the last completed update)
   __syncthreads();
   for (unsigned o = tid; o < nown; o += BS) A.x[3 * (unsigned)c0 + o] = xl[o];
+  }
+  }
 }
 
 // Empties the exchange buffers and the flag ahead of a solve.
 template <typename W>
 __global__ __launch_bounds__(256) void k_cg_resident_clear(W* q, long nq, W empty, U64* parts,
-                                                           long np, int* flag) {
+                                                           long np, int* flag, double* x, long nx) {
   const long i0 = blockIdx.x * 256L + threadIdx.x, step = gridDim.x * 256L;
   for (long i = i0; i < nq; i += step) q[i] = empty;
+  for (long i = i0; i < nx; i += step) x[i] = 0.0;  // systems that are not solved
   for (long i = i0; i < np; i += step) parts[i] = kEmpty64;
   if (i0 == 0) *flag = 0;
 }
@@ -574,6 +622,10 @@ int max_passes(int max_row, int value_bytes) {
   return max_row <= 8 ? (f32 ? 16 : 8) : max_row <= 16 ? (f32 ? 11 : 5) : f32 ? 4 : 2;
 }
 int lane_group(int max_row) { return max_row > 32 ? 16 : 8; }
+bool needs_spill(int R, int max_row, int value_bytes) {
+  const int U = max_row <= 8 ? 1 : max_row <= 16 ? 2 : 4;
+  return R * U > (value_bytes == 4 ? 12 : 6);
+}
 
 }  // namespace
 
@@ -597,21 +649,25 @@ CgResidentPlan cg_resident_plan(int nrows, int max_row, int value_bytes) {
   }
   const int rows = (nrows + P.nwg - 1) / P.nwg;
   const int passes = (int)((rows + per_pass - 1) / per_pass);
-  const int U = max_row <= 8 ? 1 : max_row <= 16 ? 2 : 4;
-  if (passes * U > (value_bytes == 4 ? 12 : 6))
+  if (needs_spill(passes, max_row, value_bytes))
     P.spill = 9L * kCgResidentSpill * kBS * P.nwg;
   return P;
 }
 
+namespace {
+
 template <typename T>
-bool launch_cg_resident(const CgResidentArgs<T>& A, int nwg, int max_row, hipStream_t st) {
+void clear(const CgResidentArgs<T>& A, hipStream_t st) {
   using W = typename std::remove_pointer<decltype(A.q)>::type;
-  const long nq = 9L * A.nrows, np = 3L * 8 * kCgResidentMaxWg;
-  const int gc = (int)std::min<long>(256, (std::max(nq, np) + 255) / 256);
+  const long nq = 9L * A.nrows, np = (A.sys ? 2L : 1L) * 3 * 8 * kCgResidentMaxWg;
+  const int gc = (int)std::min<long>(1024, (std::max(nq, np) + 255) / 256);
   hipLaunchKernelGGL(k_cg_resident_clear<W>, dim3(gc), dim3(256), 0, st, A.q, nq, Word<T>::kEmpty,
-                     A.parts, np, A.flag);
-  const int rows = (A.nrows + nwg - 1) / nwg;  // the most rows a workgroup gets
-  const int per_pass = kBS / lane_group(max_row), R = (rows + per_pass - 1) / per_pass;
+                     A.parts, np, A.flag, A.x, A.sys ? 3L * A.nrows : 0L);
+}
+
+// The kernel for R passes of rows of at most max_row blocks on nwg workgroups.
+template <typename T>
+bool launch_passes(const CgResidentArgs<T>& A, int nwg, int R, int max_row, hipStream_t st) {
   constexpr bool f32 = sizeof(T) == 4;
   // <lanes per row, blocks per lane, passes, blocks in registers, in LDS, columns
   // per thread / 3>: register counts that do not spill to scratch
@@ -655,6 +711,48 @@ bool launch_cg_resident(const CgResidentArgs<T>& A, int nwg, int max_row, hipStr
   }
   return false;
 }
+
+}  // namespace
+
+template <typename T>
+bool launch_cg_resident(const CgResidentArgs<T>& A, int nwg, int max_row, hipStream_t st) {
+  clear(A, st);
+  const int rows = (A.nrows + nwg - 1) / nwg;  // the most rows a workgroup gets
+  const int per_pass = kBS / lane_group(max_row);
+  return launch_passes(A, nwg, (rows + per_pass - 1) / per_pass, max_row, st);
+}
+
+// Teams: a system of up to 8 * 128 rows takes a team of 8 workgroups, a larger
+// one the 32 of an XCD. (An iteration costs 3-5 us in either, so small systems
+// run four to an XCD; with few systems every one takes 32, as there is room.)
+int cg_team_of(int rows, int nsys) {
+  return rows <= kCgTeamSmall * 128 && nsys > 8 ? kCgTeamSmall : kCgTeamLarge;
+}
+
+int cg_resident_batch_passes(const int* row0, int nsys, int max_row, int value_bytes, long* spill) {
+  *spill = 0;
+  if (max_row <= 0 || max_row > 64) return 0;
+  const int per_pass = kBS / lane_group(max_row);
+  int R = 0;
+  for (int b = 0; b < nsys; ++b) {
+    const int rows = row0[b + 1] - row0[b], w = cg_team_of(rows, nsys);
+    R = std::max(R, ((rows + w - 1) / w + per_pass - 1) / per_pass);
+  }
+  if (R > max_passes(max_row, value_bytes)) return 0;
+  if (needs_spill(R, max_row, value_bytes))
+    *spill = 9L * kCgResidentSpill * kBS * kCgResidentMaxWg;
+  return R;
+}
+
+template <typename T>
+bool launch_cg_resident_batch(const CgResidentArgs<T>& A, int passes, int max_row,
+                              hipStream_t st) {
+  clear(A, st);
+  return launch_passes(A, kCgResidentMaxWg, passes, max_row, st);
+}
+template bool launch_cg_resident_batch<double>(const CgResidentArgs<double>&, int, int,
+                                               hipStream_t);
+template bool launch_cg_resident_batch<float>(const CgResidentArgs<float>&, int, int, hipStream_t);
 template bool launch_cg_resident<double>(const CgResidentArgs<double>&, int, int, hipStream_t);
 template bool launch_cg_resident<float>(const CgResidentArgs<float>&, int, int, hipStream_t);
 

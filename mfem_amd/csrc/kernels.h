@@ -209,6 +209,10 @@ void launch_pcg_iteration(const PcgBuffers<T>& B, int it, hipStream_t st);
 
 // CG with the system resident in registers, one cooperative launch per solve
 // (k_cg_resident.hip): systems whose blocks fit the chip's registers.
+struct CgResidentSys {  // one of several systems: block rows [row0, row1)
+  int row0, row1, max_iters, id;
+  double tol;
+};
 template <typename T>
 struct CgResidentArgs {
   int nrows = 0;  // block rows
@@ -221,13 +225,19 @@ struct CgResidentArgs {
   double tol = 0.0;
   int max_iters = 0;
   typename std::conditional<sizeof(T) == 4, unsigned, unsigned long long>::type* q = nullptr;  // 9 nrows words
-  unsigned long long* parts = nullptr;  // 24 kCgResidentMaxWg words
+  unsigned long long* parts = nullptr;  // 24 kCgResidentMaxWg words (48 with sys)
   T* spill = nullptr;          // CgResidentPlan::spill values
   int stride = 1;              // CgResidentPlan::stride
   int lds = 0;                 // dynamic LDS of a workgroup (set by the launch)
   int* flag = nullptr;
   PcgCtrl* ctrl = nullptr;
   PcgCtrl* mirror = nullptr;   // as in PcgBuffers; its done is kCgDone or kCgExpired
+  // several systems: their list, in the order of the teams that solve them, and
+  // where each team's part begins: 9 entries for the teams of kCgTeamLarge
+  // workgroups, then 33 for those of kCgTeamSmall. ctrl and mirror are arrays
+  // then, indexed by id; x of the rows that no system covers becomes 0.
+  const CgResidentSys* sys = nullptr;
+  const int* team = nullptr;
   long long wait_ticks = 0;    // longest wait of a workgroup for the others (wall clock)
 };
 constexpr int kCgDone = 1;
@@ -243,6 +253,14 @@ struct CgResidentPlan {
   long spill = 0;
 };
 CgResidentPlan cg_resident_plan(int nrows, int max_row, int value_bytes);
+constexpr int kCgTeamLarge = 32, kCgTeamSmall = 8;
+// Workgroups of the team that solves a system of `rows` block rows among nsys.
+int cg_team_of(int rows, int nsys);
+// Passes for launch_cg_resident_batch on the systems [row0[b], row0[b + 1]), or
+// 0 where one does not fit its team, and the size of CgResidentArgs::spill.
+int cg_resident_batch_passes(const int* row0, int nsys, int max_row, int value_bytes, long* spill);
+template <typename T>
+bool launch_cg_resident_batch(const CgResidentArgs<T>& A, int passes, int max_row, hipStream_t st);
 // One solve (clears the exchange buffers first). False when the launch was
 // refused.
 template <typename T>

@@ -202,3 +202,27 @@ def test_caller_matrices(native, n):
     assert np.isfinite(x).all() and it < 20000 and rr < tol
     assert abs(true - rr) < 1e-14 * np.abs(vals).sum((1, 2)).max() * np.linalg.norm(x) / np.linalg.norm(b) * max(it, 1)
     assert not np.any(x[bare])
+
+
+# with up to 8 beams each takes the 32 workgroups of an XCD, with more the
+# small ones (up to 1024 rows) share it in teams of 8; (60, 13, 13) is past the
+# FP64 kernels' rows and sends that batch to the lockstep CG
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("sizes", [[(2, 1, 1)], [(20, 6, 6), (5, 2, 3), (33, 9, 8)],
+                                   [(4 + k, 2 + k % 5, 2 + k % 7) for k in range(21)] +
+                                   [(32, 5, 4), (31, 5, 4), (40, 11, 12), (50, 13, 12)],
+                                   [(60, 13, 13), (12, 3, 3)]])
+def test_batches(native, sizes, precision):
+    kw = dict(itr_tol=1e-12 if precision == "fp64" else 1e-10, max_iters=20000, max_newton=3)
+    scs = [scenes.beam_scene(*n, seed=k, E=10.0 ** (4 + k % 4), nu=0.3 + 0.02 * (k % 8), mixed=True,
+                             **kw) for k, n in enumerate(sizes)]
+    a, b = native.Batch(scs, precision=precision), native.Batch(scs, precision=precision)
+    b.set_cg_shape(0, 64)
+    for step in range(2):
+        a.step()
+        b.step()
+        for k in range(a.count):
+            xa, xb = a.positions(k), b.positions(k)
+            # both converge to the same dx (1e-8 of it, see the bars above);
+            # positions are of the order of the beam
+            assert np.abs(xa - xb).max() < 1e-8 * np.abs(xb).max(), (step, k)
