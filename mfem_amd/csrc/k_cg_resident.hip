@@ -20,7 +20,7 @@
 //
 // Measured on MI355X, us per iteration against the one-kernel-per-iteration CG:
 // 468 rows FP64 2.9 (8.1), 4840 rows FP64 3.5 (9.2), 37.5k rows FP64 5.2 (16),
-// 54.8k rows FP32 6.5 (13.2), 168k rows FP32 20 (26). What is left of a small
+// 54.8k rows FP32 6.5 (13.2), 168k rows FP32 15 (26). What is left of a small
 // system's 2.9 us is the exchange (0.6 us on one XCD, 1-2 us over all), three
 // workgroup barriers, two chains of wave sums, the two divisions and the loads
 // of q.
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   constexpr int kAcc = 3 * (BS / G);
   constexpr int kPolls = kCgResidentMaxWg / kWave;
   using L = ResidentLds<R, NLDS, EPT, BS, G, T>;
-  static_assert(NP <= BS / kWave, "one wave per sum");
+  constexpr int NW = BS / kWave;
   extern __shared__ __align__(16) unsigned char dyn[];
   __shared__ double s_acc[NP][BS / 4 > kAcc ? BS / 4 : kAcc];
   __shared__ double s_tot[NP];
@@ -396,9 +396,9 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
         if (m * BS < nent && e < nent && e - own0 >= nown)
           w[m] = word_load(word_at(qv, 3 * list[e / 3] + e % 3));
       }
-      // sum `wid` of iteration it-1 over the workgroups
-      if (wid < kCgParts || (wid == kCgParts && it == 1)) {
-        const U64* src = parts + ((size_t)prev * kCgResidentMaxWg + g0) * 8 + wid;
+      // sums of iteration it-1 over the workgroups, one per wave at a time
+      for (int k = wid; k < (it == 1 ? NP : kCgParts); k += NW) {
+        const U64* src = parts + ((size_t)prev * kCgResidentMaxWg + g0) * 8 + k;
         U64 s[kPolls];
 #pragma unroll
         for (int h = 0; h < kPolls; ++h) {
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
           v += __builtin_bit_cast(double, s[h]);
         }
         v = wave_sum_63(v);
-        if ((tid & (kWave - 1)) == kWave - 1) s_tot[wid] = v;
+        if ((tid & (kWave - 1)) == kWave - 1) s_tot[k] = v;
       }
       if (dead) s_dead = 1;
       __syncthreads();
@@ -491,46 +491,43 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
     }
     if (dead) s_dead = 1;  // seen behind the barriers below
     __syncthreads();
-    T q[R];
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-      q[j] = (T)0;
-      if (R > 1 && j * (BS / G) >= rows) continue;  // no rows in this pass
-      // one pass's loads at a time where registers are short
-      if constexpr (NSTR > 0 || NLDS > 0) asm volatile("" ::: "memory");
-      T y0 = 0, y1 = 0, y2 = 0;
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = j * U + u;
-        const T* p = reinterpret_cast<const T*>(
-            reinterpret_cast<const unsigned char*>(pl) + ((off[i / 2] >> (16 * (i & 1))) & 0xffff));
-        T v[9];
-        unsigned ks = i < NREG + NLDS ? 0 : opaque((i - NREG - NLDS) * 9 * BS + tid);
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-          v[k] = i < NREG ? V[i < NREG ? i : 0][k]
-                 : i < NREG + NLDS ? vl[((i - NREG) * 9 + k) * BS + tid]
-                                   : *word_at(vs, ks);
-          ks += BS;
-        }
-        const T p0 = p[0], p1 = p[1], p2 = p[2];
-        y0 += v[0] * p0 + v[1] * p1 + v[2] * p2;
-        y1 += v[3] * p0 + v[4] * p1 + v[5] * p2;
-        y2 += v[6] * p0 + v[7] * p1 + v[8] * p2;
-      }
-      q[j] = group_sum3<G>(y0, y1, y2, lane);
-    }
-    // the resets of this iteration are complete before anything of it is
-    // published
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    // q = K p, published pass by pass
     W* now = A.q + (size_t)slot * n;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
+      T y0 = 0, y1 = 0, y2 = 0;
+      if (R == 1 || j * (BS / G) < rows) {  // the pass has rows
+        // one pass's loads at a time where registers are short
+        if constexpr (NSTR > 0 || NLDS > 0) asm volatile("" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int i = j * U + u;
+          const T* p = reinterpret_cast<const T*>(reinterpret_cast<const unsigned char*>(pl) +
+                                                  ((off[i / 2] >> (16 * (i & 1))) & 0xffff));
+          T v[9];
+          unsigned ks = i < NREG + NLDS ? 0 : opaque((i - NREG - NLDS) * 9 * BS + tid);
+#pragma unroll
+          for (int k = 0; k < 9; ++k) {
+            v[k] = i < NREG ? V[i < NREG ? i : 0][k]
+                   : i < NREG + NLDS ? vl[((i - NREG) * 9 + k) * BS + tid]
+                                     : *word_at(vs, ks);
+            ks += BS;
+          }
+          const T p0 = p[0], p1 = p[1], p2 = p[2];
+          y0 += v[0] * p0 + v[1] * p1 + v[2] * p2;
+          y1 += v[3] * p0 + v[4] * p1 + v[5] * p2;
+          y2 += v[6] * p0 + v[7] * p1 + v[8] * p2;
+        }
+      }
+      const T q = group_sum3<G>(y0, y1, y2, lane);
+      // the resets of this iteration are complete before anything of it is
+      // published
+      if (j == 0) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
       const unsigned o = 3 * (j * (BS / G) + tid / G) + lane;
       if (lane < 3 && o < nown) {
-        word_store(word_at(now, 3 * (unsigned)c0 + o), __builtin_bit_cast(W, q[j]));
-        ql[o] = q[j];
-        const double dq = (double)q[j];
+        word_store(word_at(now, 3 * (unsigned)c0 + o), __builtin_bit_cast(W, q));
+        ql[o] = q;
+        const double dq = (double)q;
         acc[0] += (double)pl[own0 + o] * dq;
         acc[1] += (double)zl[o] * dq;
         acc[2] += dq * ((double)dl[o] * dq);
@@ -550,17 +547,17 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
     }
     __syncthreads();
     if (s_dead) break;
-    if (wid < kCgParts || (wid == kCgParts && it == 0)) {
+    for (int k = wid; k < (it == 0 ? NP : kCgParts); k += NW) {
       double t = 0.0;
-      const int m = wid < 3 ? kAcc : BS / 4;
+      const int m = k < 3 ? kAcc : BS / 4;
 #pragma unroll
       for (int o = 0; o < (kAcc > BS / 4 ? kAcc : BS / 4); o += kWave) {
         const int i = o + (tid & (kWave - 1));
-        t += i < m ? s_acc[wid][i] : 0.0;
+        t += i < m ? s_acc[k][i] : 0.0;
       }
       t = wave_sum_63(t);
       if ((tid & (kWave - 1)) == kWave - 1)
-        word_store(parts + ((size_t)slot * kCgResidentMaxWg + g0 + wg) * 8 + wid,
+        word_store(parts + ((size_t)slot * kCgResidentMaxWg + g0 + wg) * 8 + k,
                    __builtin_bit_cast(U64, t));
     }
     used = used || it > 0 || si > s0;
@@ -594,24 +591,25 @@ __global__ __launch_bounds__(256) void k_cg_resident_clear(W* q, long nq, W empt
   if (i0 == 0) *flag = 0;
 }
 
-constexpr int kBS = 512;
+constexpr int kBS = 512;  // threads of a workgroup (kBigBS for the largest systems)
+constexpr int kBigBS = 256;
 constexpr int kLdsBytes = 150 * 1024;  // dynamic LDS of a workgroup (one per CU)
 
-template <int G, int U, int R, int NREG, int NLDS, int EPT, typename T>
+template <int G, int U, int R, int NREG, int NLDS, int EPT, int BS = kBS, typename T>
 bool launch_shape(const CgResidentArgs<T>& A, int nwg, hipStream_t st) {
   static_assert(NREG + NLDS + kCgResidentSpill >= R * U, "spill area");
-  using L = ResidentLds<R, NLDS, EPT, kBS, G, T>;
+  using L = ResidentLds<R, NLDS, EPT, BS, G, T>;
   static_assert(L::p < kLdsBytes, "LDS");
   if (NREG + NLDS < R * U && !A.spill) return false;
   if (L::start + 8L * ((A.nrows + 31) / 32) > kLdsBytes) return false;
   const void* f = reinterpret_cast<const void*>(
-      &k_cg_resident<G, U, R, NREG, NLDS, EPT, kBS, T>);
+      &k_cg_resident<G, U, R, NREG, NLDS, EPT, BS, T>);
   if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess)
     return false;
   CgResidentArgs<T> a = A;
   a.lds = kLdsBytes;
   void* args[] = {&a};
-  return hipLaunchCooperativeKernel(f, dim3(nwg * A.stride), dim3(kBS), args, kLdsBytes, st) ==
+  return hipLaunchCooperativeKernel(f, dim3(nwg * A.stride), dim3(BS), args, kLdsBytes, st) ==
          hipSuccess;
 }
 
@@ -622,9 +620,10 @@ int max_passes(int max_row, int value_bytes) {
   return max_row <= 8 ? (f32 ? 16 : 8) : max_row <= 16 ? (f32 ? 11 : 5) : f32 ? 4 : 2;
 }
 int lane_group(int max_row) { return max_row > 32 ? 16 : 8; }
+// more passes than the kernels without blocks in A.spill have
 bool needs_spill(int R, int max_row, int value_bytes) {
-  const int U = max_row <= 8 ? 1 : max_row <= 16 ? 2 : 4;
-  return R * U > (value_bytes == 4 ? 12 : 6);
+  const bool f32 = value_bytes == 4;
+  return R > (max_row <= 8 ? (f32 ? 8 : 4) : max_row <= 16 ? (f32 ? 6 : 3) : (f32 ? 2 : 1));
 }
 
 }  // namespace
@@ -670,14 +669,17 @@ template <typename T>
 bool launch_passes(const CgResidentArgs<T>& A, int nwg, int R, int max_row, hipStream_t st) {
   constexpr bool f32 = sizeof(T) == 4;
   // <lanes per row, blocks per lane, passes, blocks in registers, in LDS, columns
-  // per thread / 3>: register counts that do not spill to scratch
+  // per thread / 3>. A register spilled to scratch costs an iteration as much as
+  // a block value in A.spill and more latency, so the counts are the largest
+  // that spill none or next to none: for 11 passes in FP32, 8 blocks in
+  // registers take 15.0 us an iteration at 168k rows, 10 take 16.7, 11 took 18.4.
   if (max_row <= 8) {
     if (R <= 1) return launch_shape<8, 1, 1, 1, 0, 8>(A, nwg, st);
     if (R <= 2) return launch_shape<8, 1, 2, 2, 0, 8>(A, nwg, st);
     if (R <= 4) return launch_shape<8, 1, 4, 4, 0, 8>(A, nwg, st);
     if constexpr (f32) {
       if (R <= 8) return launch_shape<8, 1, 8, 8, 0, 12>(A, nwg, st);
-      if (R <= 16) return launch_shape<8, 1, 16, 9, 3, 14>(A, nwg, st);
+      if (R <= 16) return launch_shape<8, 1, 16, 7, 3, 14>(A, nwg, st);
     } else {
       if (R <= 8) return launch_shape<8, 1, 8, 4, 2, 8>(A, nwg, st);
     }
@@ -687,7 +689,7 @@ bool launch_passes(const CgResidentArgs<T>& A, int nwg, int R, int max_row, hipS
     if constexpr (f32) {
       if (R <= 4) return launch_shape<8, 2, 4, 8, 0, 8>(A, nwg, st);
       if (R <= 6) return launch_shape<8, 2, 6, 9, 3, 12>(A, nwg, st);
-      if (R <= 11) return launch_shape<8, 2, 11, 11, 3, 14>(A, nwg, st);
+      if (R <= 11) return launch_shape<8, 2, 11, 8, 3, 14>(A, nwg, st);
     } else {
       if (R <= 3) return launch_shape<8, 2, 3, 4, 2, 8>(A, nwg, st);
       if (R <= 5) return launch_shape<8, 2, 5, 4, 2, 8>(A, nwg, st);

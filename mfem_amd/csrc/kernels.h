@@ -244,7 +244,7 @@ constexpr int kCgDone = 1;
 constexpr int kCgExpired = 2;  // a wait expired: there is no solution
 constexpr int kCgNoFit = 3;    // a workgroup's columns do not fit: there is no solution
 constexpr int kCgResidentMaxWg = 256;
-constexpr int kCgResidentSpill = 8;  // most blocks of a lane in `spill`
+constexpr int kCgResidentSpill = 12;  // most blocks of a lane in `spill`
 // Workgroups that the resident CG takes for nrows block rows of at most
 // max_row blocks (0: the system does not fit), and the values that
 // CgResidentArgs::spill needs (0: none).
