@@ -1312,52 +1312,87 @@ __global__ __launch_bounds__(kElemBlock) void k_plain2d_energy(
 
 // ---------------------------------------------------------------------------
 // Batched element evaluations (points in AoS, column-major per point).
-__global__ void k_batch_polar(int n, const double* __restrict__ F, double* __restrict__ R,
-                              double* __restrict__ s, double* __restrict__ dsdF,
-                              int* __restrict__ iters) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// Records of the batched entry points (element-major, N values each) pass
+// through LDS, so that a wave reads and writes contiguous runs: from every lane
+// a record of its own would touch 64 cache lines per instruction. An odd pitch
+// keeps the LDS banks apart. One wave per workgroup.
+template <int N>
+constexpr int kRecPitch = N | 1;
+
+template <int N>
+__device__ __forceinline__ void record_in(const double* __restrict__ src, int e0, int n,
+                                          double* lds, double (&v)[N]) {
+  const int lane = threadIdx.x, m = min(kWave, n - e0) * N;
+  __syncthreads();
+  for (int i = lane; i < m; i += kWave) lds[(i / N) * kRecPitch<N> + i % N] = src[(size_t)e0 * N + i];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = e0 + lane < n ? lds[lane * kRecPitch<N> + k] : 0.0;
+}
+// (half a wave's records at a time: half the LDS, twice the workgroups per CU)
+template <int N>
+__device__ __forceinline__ void record_out(const double (&v)[N], int e0, int n, double* lds,
+                                           double* __restrict__ dst) {
+  const int lane = threadIdx.x;
+#pragma unroll 1
+  for (int h = 0; h < 2; ++h) {
+    const int b = e0 + h * (kWave / 2);
+    __syncthreads();
+    if (lane / (kWave / 2) == h)
+#pragma unroll
+      for (int k = 0; k < N; ++k) lds[(lane & (kWave / 2 - 1)) * kRecPitch<N> + k] = v[k];
+    __syncthreads();
+    const int m = min(kWave / 2, n - b) * N;
+    for (int i = lane; i < m; i += kWave) dst[(size_t)b * N + i] = lds[(i / N) * kRecPitch<N> + i % N];
+  }
+}
+
+__global__ __launch_bounds__(kWave) void k_batch_polar(int n, const double* __restrict__ F,
+                                                       double* __restrict__ R,
+                                                       double* __restrict__ s,
+                                                       double* __restrict__ dsdF,
+                                                       int* __restrict__ iters) {
+  __shared__ double lds[kWave / 2 * kRecPitch<54>];
+  static_assert(kWave * kRecPitch<9> <= kWave / 2 * kRecPitch<54>, "LDS");
+  const int e0 = blockIdx.x * kWave, i = e0 + threadIdx.x;
   double Fl[9], Rl[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) { Fl[k] = F[9 * i + k]; Rl[k] = R[9 * i + k]; }
-  int it = procrustes(Rl, Fl, 1e-6, 100);
+  record_in<9>(F, e0, n, lds, Fl);
+  record_in<9>(R, e0, n, lds, Rl);
   double Sm[9], sv[6];
+  int it = 0;
+  if (i < n) it = procrustes(Rl, Fl, 1e-6, 100);
   stretch_of(Rl, Fl, sv, Sm);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) R[9 * i + k] = Rl[k];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) s[6 * i + k] = sv[k];
+  record_out<9>(Rl, e0, n, lds, R);
+  record_out<6>(sv, e0, n, lds, s);
   if (dsdF) {
     double d[54];
     dsdF_of<double>(Rl, Fl, d);
-#pragma unroll
-    for (int k = 0; k < 54; ++k) dsdF[54 * i + k] = d[k];
+    record_out<54>(d, e0, n, lds, dsdF);
   }
-  if (iters) iters[i] = it;
+  if (iters && i < n) iters[i] = it;
 }
 
-__global__ void k_batch_material(int n, const int* __restrict__ type, const double* __restrict__ mu,
-                                 const double* __restrict__ la, const double* __restrict__ s,
-                                 int psd, double* __restrict__ E, double* __restrict__ g,
-                                 double* __restrict__ H) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+__global__ __launch_bounds__(kWave) void k_batch_material(
+    int n, const int* __restrict__ type, const double* __restrict__ mu,
+    const double* __restrict__ la, const double* __restrict__ s, int psd, double* __restrict__ E,
+    double* __restrict__ g, double* __restrict__ H) {
+  __shared__ double lds[kWave / 2 * kRecPitch<36>];
+  static_assert(kWave * kRecPitch<6> <= kWave / 2 * kRecPitch<36>, "LDS");
+  const int e0 = blockIdx.x * kWave, i = e0 + threadIdx.x, ic = min(i, n - 1);
   double sv[6];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) sv[k] = s[6 * i + k];
-  if (E) E[i] = material_energy(type[i], mu[i], la[i], sv);
+  record_in<6>(s, e0, n, lds, sv);
+  const int t = type[ic];
+  if (E && i < n) E[i] = material_energy(t, mu[i], la[i], sv);
   double gg[6], HH[21];
-  material_grad_hess(type[i], mu[i], la[i], sv, gg, HH);
-  if (psd && material_needs_psd(type[i]) && !chol_pd_packed<double, 6>(HH, 1e-6))
+  material_grad_hess(t, mu[ic], la[ic], sv, gg, HH);
+  if (psd && i < n && material_needs_psd(t) && !chol_pd_packed<double, 6>(HH, 1e-6))
     jacobi_psd_project_packed<double, 6>(HH, 1e-6);
-  double A[36];
-  unpack_sym6(HH, A);
-  if (g)
-#pragma unroll
-    for (int k = 0; k < 6; ++k) g[6 * i + k] = gg[k];
-  if (H)
-#pragma unroll
-    for (int k = 0; k < 36; ++k) H[36 * i + k] = A[k];
+  if (g) record_out<6>(gg, e0, n, lds, g);
+  if (H) {
+    double A[36];
+    unpack_sym6(HH, A);
+    record_out<36>(A, e0, n, lds, H);
+  }
 }
 
 __global__ void k_batch_snh_f9(int n, const double* __restrict__ mu, const double* __restrict__ la,
