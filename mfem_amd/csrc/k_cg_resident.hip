@@ -591,8 +591,7 @@ __global__ __launch_bounds__(256) void k_cg_resident_clear(W* q, long nq, W empt
   if (i0 == 0) *flag = 0;
 }
 
-constexpr int kBS = 512;  // threads of a workgroup (kBigBS for the largest systems)
-constexpr int kBigBS = 256;
+constexpr int kBS = 512;  // threads of a workgroup
 constexpr int kLdsBytes = 150 * 1024;  // dynamic LDS of a workgroup (one per CU)
 
 template <int G, int U, int R, int NREG, int NLDS, int EPT, int BS = kBS, typename T>
@@ -634,17 +633,21 @@ bool needs_spill(int R, int max_row, int value_bytes) {
 // workgroup of the launch), whose L2 they share: 468 rows in FP64 take 2.9 us
 // an iteration on 16 workgroups of one XCD, 3.9 us on 64 over all of them; 4840
 // rows 4.5 us on the 32 of one XCD, 3.4 us on 96.
+// 31 of an XCD's 32 CUs at most: kernels of other streams still find a CU while
+// a solve spins (256 instead of 248 workgroups gained nothing: 15.0 us an
+// iteration at 168k rows either way).
 CgResidentPlan cg_resident_plan(int nrows, int max_row, int value_bytes) {
+  constexpr int kMaxWg = kCgResidentMaxWg / 32 * 31;
   CgResidentPlan P;
   if (nrows <= 0 || max_row <= 0 || max_row > 64) return P;
   const long per_pass = kBS / lane_group(max_row);
-  const long most = kCgResidentMaxWg * per_pass * max_passes(max_row, value_bytes);
+  const long most = kMaxWg * per_pass * max_passes(max_row, value_bytes);
   if (nrows > most) return P;
   if (nrows <= 32 * per_pass) {
     P.stride = 8;
     P.nwg = (int)std::min<long>(32, (nrows + 31) / 32);
   } else {
-    P.nwg = (int)std::min<long>(kCgResidentMaxWg, (nrows + 8 * 50 - 1) / (8 * 50) * 8);
+    P.nwg = (int)std::min<long>(kMaxWg, (nrows + 8 * 50 - 1) / (8 * 50) * 8);
   }
   const int rows = (nrows + P.nwg - 1) / P.nwg;
   const int passes = (int)((rows + per_pass - 1) / per_pass);
