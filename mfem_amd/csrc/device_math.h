@@ -73,7 +73,78 @@ MFEM_DEV void rodrigues(const double w[3], double dR[9]) {
   dR[7] = -sn * kx + oc * ky * kz;  // (1,2)
 }
 
+// -tr(dR Y) of the rotation dR about w
+MFEM_DEV double procrustes_trial(const double w[3], const double Y[9], double dR[9]) {
+  rodrigues(w, dR);
+  double t = 0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) t += dR[i + 3 * k] * Y[k + 3 * i];
+  return -t;
+}
+
+// Further trials of the lanes with `more`, all lanes of the wave helping: with n
+// such lanes, lane l evaluates trial l / n of the (l % n)-th one (0.6^j w), and
+// each takes the first trial that the rule accepts. dR is its rotation.
+MFEM_DEV void procrustes_shared_trials(double w[3], const double Y[9], double E0, double tol,
+                                       bool more, unsigned long long slow, double dR[9]) {
+  const unsigned long long act = __ballot(true);
+  const bool mine = more;
+  if (act & (act + 1)) {  // the active lanes are no prefix of the wave: each by itself
+    while (more) {
+      const double E1 = procrustes_trial(w, Y, dR);
+      w[0] *= 0.6; w[1] *= 0.6; w[2] *= 0.6;
+      more = E1 > E0 && sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]) > tol;
+    }
+    return;
+  }
+  const int self = (int)(threadIdx.x & 63), lanes = __popcll(act);
+  const unsigned long long below = (1ull << self) - 1;
+  while (slow) {  // the same for every lane
+    const int n = __popcll(slow), rank = __popcll(slow & below);
+    // lane q < n learns which lane is the q-th slow one
+    const int to = more ? rank : n + __popcll(~slow & act & below);
+    const int src = __shfl(__builtin_amdgcn_ds_permute(4 * to, self), self % n);
+    double f = 1.0, b = 0.6;  // 0.6^j
+    for (int j = self / n; j; j >>= 1, b *= b)
+      if (j & 1) f *= b;
+    double t[3], Yc[9], d[9];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) t[i] = __shfl(w[i], src) * f;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) Yc[i] = __shfl(Y[i], src);
+    const double Ec = __shfl(E0, src);
+    const double E1 = procrustes_trial(t, Yc, d);
+    const double u[3] = {t[0] * 0.6, t[1] * 0.6, t[2] * 0.6};
+    const unsigned long long ok =
+        __ballot(!(E1 > Ec && sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]) > tol));
+    int at = self;  // the accepted trial's lane, or the last trial's
+    bool found = false;
+    if (more)
+      for (int l = rank; l < lanes && !found; l += n) {
+        at = l;
+        found = (ok >> l) & 1;
+      }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const double s = __shfl(t[i], at);
+      if (more) w[i] = found ? s : s * 0.6;
+    }
+    more = more && !found;
+    slow = __ballot(more);
+  }
+  if (mine) rodrigues(w, dR);
+}
+
 // R (in: warm start, out: rotation), F column-major. Returns iterations.
+//
+// Called by any set of lanes of a wave, which leave together. Almost every fit
+// accepts its first trial or two, but an element far from its warm start (a step
+// of an unconverged solve) can shrink its step to the tolerance in every one of
+// 100 iterations, some 25 trials each, while the other lanes wait. A serial
+// chain of FP64 sin/cos bounds such a wave, so from the third trial on its lanes
+// share them: the energy of 304k tets at such a step takes 1020 us instead of 2210.
 MFEM_DEV int procrustes(double R[9], const double F[9], double tol, int max_iter) {
   double Y[9];
   // Y = R F^T
@@ -83,42 +154,49 @@ MFEM_DEV int procrustes(double R[9], const double F[9], double tol, int max_iter
     for (int r = 0; r < 3; ++r)
       Y[r + 3 * c] = R[r] * F[c] + R[r + 3] * F[c + 3] + R[r + 6] * F[c + 6];
   int itr = 0;
-  do {
-    double g[3] = {Y[5] - Y[7], Y[6] - Y[2], Y[1] - Y[3]};
-    if (sqrt(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]) < tol) break;
-    double tr = Y[0] + Y[4] + Y[8];
-    double H[6] = {tr - Y[0], tr - Y[4], tr - Y[8], -0.5 * (Y[3] + Y[1]),
-                   -0.5 * (Y[6] + Y[2]), -0.5 * (Y[7] + Y[5])};
-    double w[3];
-    solve3_sym(H, g, w);
-    w[0] = -w[0]; w[1] = -w[1]; w[2] = -w[2];
-    // E0 = -tr(R Y)
-    double trRY = 0;
+  bool live = true;
+  for (;;) {
+    double w[3] = {0, 0, 0}, dR[9], E0 = 0;
+    bool more = false;  // the rule asks for another, smaller trial
+    if (live) {
+      double g[3] = {Y[5] - Y[7], Y[6] - Y[2], Y[1] - Y[3]};
+      live = !(sqrt(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]) < tol);
+      if (live) {
+        double tr = Y[0] + Y[4] + Y[8];
+        double H[6] = {tr - Y[0], tr - Y[4], tr - Y[8], -0.5 * (Y[3] + Y[1]),
+                       -0.5 * (Y[6] + Y[2]), -0.5 * (Y[7] + Y[5])};
+        solve3_sym(H, g, w);
+        w[0] = -w[0]; w[1] = -w[1]; w[2] = -w[2];
+        // E0 = -tr(R Y)
+        double trRY = 0;
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+        for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) trRY += R[i + 3 * k] * Y[k + 3 * i];
-    double E0 = -trRY, E1;
-    double dR[9];
-    do {
-      rodrigues(w, dR);
-      double t = 0;
+          for (int k = 0; k < 3; ++k) trRY += R[i + 3 * k] * Y[k + 3 * i];
+        E0 = -trRY;
+        double E1;
+        int n = 0;
+        do {
+          E1 = procrustes_trial(w, Y, dR);
+          w[0] *= 0.6; w[1] *= 0.6; w[2] *= 0.6;
+          more = E1 > E0 && sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]) > tol;
+        } while (more && ++n < 2);
+      }
+    }
+    if (!__any(live)) break;
+    unsigned long long slow = __ballot(more);
+    if (slow) procrustes_shared_trials(w, Y, E0, tol, more, slow, dR);
+    if (live) {
+      double T1[9];
+      matmul3(dR, R, T1);
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
+      for (int i = 0; i < 9; ++i) R[i] = T1[i];
+      matmul3(dR, Y, T1);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) t += dR[i + 3 * k] * Y[k + 3 * i];
-      E1 = -t;
-      w[0] *= 0.6; w[1] *= 0.6; w[2] *= 0.6;
-    } while (E1 > E0 && sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]) > tol);
-    double T1[9];
-    matmul3(dR, R, T1);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) R[i] = T1[i];
-    matmul3(dR, Y, T1);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Y[i] = T1[i];
-    ++itr;
-  } while (itr < max_iter);
+      for (int i = 0; i < 9; ++i) Y[i] = T1[i];
+      live = ++itr < max_iter;
+    }
+  }
   return itr;
 }
 

@@ -1,0 +1,55 @@
+"""Batched element entry points at the edges of a wave and of the half wave in
+which their records pass through LDS, and the rotation fit's shared trials (the
+lanes of a wave evaluate the trials of the elements that need many). Needs an
+MI355X.
+
+Records against the oracle with the bounds of the element-level parity tests.
+Shared trials against the same elements one to a launch, where a lane has no
+helpers: both form the same trials (0.6^j w by powers against one product after
+the other, up to 100 roundings of 1e-16) and accept by one rule, so iteration
+counts are equal and R agrees to 100 applied rotations of that rounding, 1e-12."""
+import numpy as np
+import pytest
+
+from mfem_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 63, 64, 65])
+def test_records_at_wave_edges(n, oracle):
+    from mfem_amd import native
+    rng = np.random.RandomState(n)
+    F = np.eye(3) + 0.15 * rng.uniform(-1, 1, (n, 3, 3))
+    mu, la = scenes.enu_to_lame(1e6, 0.45)
+    S = np.array([1, 1, 1, 0, 0, 0.0]) + 0.2 * rng.uniform(-1, 1, (n, 6))
+    R, s, dsdF, it = native.polar_batch(F)
+    E, g, H = native.material_s6_batch(0, mu, la, S)
+    for i in range(n):
+        Ro, so, do, _, ito = oracle.polar_svd3(F[i])
+        assert it[i] == ito
+        assert np.abs(R[i] - Ro).max() < 1e-12 and np.abs(s[i] - so).max() < 1e-12
+        assert np.abs(dsdF[i] - do).max() < 1e-10 * np.abs(do).max()
+        Eo, go, Ho = oracle.material_s6(0, mu, la, S[i], True)
+        assert abs(E[i] - Eo) <= 1e-12 * max(abs(Eo), mu)
+        assert np.abs(g[i] - go).max() <= 1e-12 * max(np.abs(go).max(), mu)
+        assert np.abs(H[i] - Ho).max() <= 1e-9 * np.abs(Ho).max(), i
+
+
+@pytest.mark.parametrize("n,wild", [(1, 1), (64, 1), (64, 64), (65, 13), (190, 40)])
+def test_shared_trials_equal_single_launches(n, wild):
+    from mfem_amd import native
+    rng = np.random.RandomState(n + wild)
+    F = np.eye(3) + 0.1 * rng.randn(n, 3, 3)
+    Q, _ = np.linalg.qr(rng.randn(n, 3, 3))
+    Q *= np.sign(np.linalg.det(Q))[:, None, None]
+    R0 = np.tile(np.eye(3), (n, 1, 1))
+    far = rng.choice(n, wild, replace=False)
+    # stretched elements whose fit is far from their warm start
+    F[far] = Q[far] @ np.diag([5.0, 2.0, 0.7]) @ np.swapaxes(np.roll(Q, 1, 0)[far], 1, 2)
+    R, s, _, it = native.polar_batch(F, R0)
+    assert np.isfinite(R).all() and (wild < 13 or it.max() > 5)
+    for e in range(n) if n <= 65 else far:
+        R1, s1, _, it1 = native.polar_batch(F[e:e + 1], R0[e:e + 1])
+        assert it1[0] == it[e], e
+        assert np.abs(R1[0] - R[e]).max() < 1e-12 and np.abs(s1[0] - s[e]).max() < 1e-11, e
