@@ -73,6 +73,55 @@ MFEM_DEV void rodrigues(const double w[3], double dR[9]) {
   dR[7] = -sn * kx + oc * ky * kz;  // (1,2)
 }
 
+// R (in: warm start, out: rotation), F column-major. Returns iterations.
+MFEM_DEV int procrustes(double R[9], const double F[9], double tol, int max_iter) {
+  double Y[9];
+  // Y = R F^T
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      Y[r + 3 * c] = R[r] * F[c] + R[r + 3] * F[c + 3] + R[r + 6] * F[c + 6];
+  int itr = 0;
+  do {
+    double g[3] = {Y[5] - Y[7], Y[6] - Y[2], Y[1] - Y[3]};
+    if (sqrt(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]) < tol) break;
+    double tr = Y[0] + Y[4] + Y[8];
+    double H[6] = {tr - Y[0], tr - Y[4], tr - Y[8], -0.5 * (Y[3] + Y[1]),
+                   -0.5 * (Y[6] + Y[2]), -0.5 * (Y[7] + Y[5])};
+    double w[3];
+    solve3_sym(H, g, w);
+    w[0] = -w[0]; w[1] = -w[1]; w[2] = -w[2];
+    // E0 = -tr(R Y)
+    double trRY = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) trRY += R[i + 3 * k] * Y[k + 3 * i];
+    double E0 = -trRY, E1;
+    double dR[9];
+    do {
+      rodrigues(w, dR);
+      double t = 0;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) t += dR[i + 3 * k] * Y[k + 3 * i];
+      E1 = -t;
+      w[0] *= 0.6; w[1] *= 0.6; w[2] *= 0.6;
+    } while (E1 > E0 && sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]) > tol);
+    double T1[9];
+    matmul3(dR, R, T1);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) R[i] = T1[i];
+    matmul3(dR, Y, T1);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) Y[i] = T1[i];
+    ++itr;
+  } while (itr < max_iter);
+  return itr;
+}
+
 // -tr(dR Y) of the rotation dR about w
 MFEM_DEV double procrustes_trial(const double w[3], const double Y[9], double dR[9]) {
   rodrigues(w, dR);
@@ -106,12 +155,12 @@ MFEM_DEV void procrustes_shared_trials(double w[3], const double Y[9], double E0
     // lane q < n learns which lane is the q-th slow one
     const int to = more ? rank : n + __popcll(~slow & act & below);
     const int src = __shfl(__builtin_amdgcn_ds_permute(4 * to, self), self % n);
-    double f = 1.0, b = 0.6;  // 0.6^j
-    for (int j = self / n; j; j >>= 1, b *= b)
-      if (j & 1) f *= b;
     double t[3], Yc[9], d[9];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) t[i] = __shfl(w[i], src) * f;
+    for (int i = 0; i < 3; ++i) t[i] = __shfl(w[i], src);
+    for (int j = self / n; j > 0; --j) {  // as the lane itself would shrink it
+      t[0] *= 0.6; t[1] *= 0.6; t[2] *= 0.6;
+    }
 #pragma unroll
     for (int i = 0; i < 9; ++i) Yc[i] = __shfl(Y[i], src);
     const double Ec = __shfl(E0, src);
@@ -137,15 +186,17 @@ MFEM_DEV void procrustes_shared_trials(double w[3], const double Y[9], double E0
   if (mine) rodrigues(w, dR);
 }
 
-// R (in: warm start, out: rotation), F column-major. Returns iterations.
-//
-// Called by any set of lanes of a wave, which leave together. Almost every fit
-// accepts its first trial or two, but an element far from its warm start (a step
-// of an unconverged solve) can shrink its step to the tolerance in every one of
-// 100 iterations, some 25 trials each, while the other lanes wait. A serial
-// chain of FP64 sin/cos bounds such a wave, so from the third trial on its lanes
-// share them: the energy of 304k tets at such a step takes 1020 us instead of 2210.
-MFEM_DEV int procrustes(double R[9], const double F[9], double tol, int max_iter) {
+// procrustes() for kernels that must stand elements far from their warm start
+// (the energy of a line-search trial, a caller's own elements). Called by any set
+// of lanes of a wave, which leave together. Almost every fit accepts its first
+// trial or two, but after a step of an unconverged solve an element can shrink
+// its step to the tolerance in every one of 100 iterations, some 25 trials each,
+// while the other lanes wait. A serial chain of FP64 sin/cos bounds such a wave,
+// so from the third trial on its lanes share them: the energy of 304k tets at
+// such a step takes 1020 us instead of 2210. Same trials and same rule as
+// procrustes(); the compiler rounds the two differently in the last place, so the
+// state update keeps that one.
+MFEM_DEV int procrustes_wave(double R[9], const double F[9], double tol, int max_iter) {
   double Y[9];
   // Y = R F^T
 #pragma unroll
@@ -176,6 +227,7 @@ MFEM_DEV int procrustes(double R[9], const double F[9], double tol, int max_iter
         E0 = -trRY;
         double E1;
         int n = 0;
+#pragma unroll 1
         do {
           E1 = procrustes_trial(w, Y, dR);
           w[0] *= 0.6; w[1] *= 0.6; w[2] *= 0.6;

@@ -616,7 +616,7 @@ __device__ __forceinline__ double mixed_energy_tet(const TetMeshDev& m, int e,
   double Rl[9];
 #pragma unroll
   for (int i = 0; i < 9; ++i) Rl[i] = R[i * nT + e];
-  procrustes(Rl, F, 1e-6, 100);
+  procrustes_wave(Rl, F, 1e-6, 100);
   double Sm[9], sv[6], sa[6];
   stretch_of(Rl, F, sv, Sm);
   double ec = 0;
@@ -1360,7 +1360,7 @@ __global__ __launch_bounds__(kWave) void k_batch_polar(int n, const double* __re
   record_in<9>(R, e0, n, lds, Rl);
   double Sm[9], sv[6];
   int it = 0;
-  if (i < n) it = procrustes(Rl, Fl, 1e-6, 100);
+  if (i < n) it = procrustes_wave(Rl, Fl, 1e-6, 100);
   stretch_of(Rl, Fl, sv, Sm);
   record_out<9>(Rl, e0, n, lds, R);
   record_out<6>(sv, e0, n, lds, s);
