@@ -21,14 +21,24 @@
 // follows Eigen 3.4's preconditioned Lanczos/Givens recurrence
 // (unsupported/Eigen/src/IterativeSolvers/MINRES.h). One iteration is
 //   k_mr_tet, k_mr_vertex   p/x update of the previous iteration; v_new = K w - beta v_old
-//   k_mr_fin_alpha          alpha = v_new . w
-//   k_mr_prec_tet, _vtx0    v_new -= alpha v; w_new = P v_new (element blocks,
-//                           first Chebyshev step of the mass block)
+//   k_mr_prec               alpha = v_new . w; v_new -= alpha v; w_new = P v_new (element
+//                           blocks, first Chebyshev step of the mass block)
 //   k_mr_cheb x 3           Chebyshev steps of the mass block
 //   k_mr_fin_beta           beta_new, Givens rotation, stopping test
 // with every scalar in one MinresCtrl block on the device. Lanczos vectors are
 // stored unnormalised: v_k = V_k / beta_k, w_k = W_k / beta_k. Every sum is a
-// per-workgroup partial reduced in index order by a one-workgroup kernel.
+// per-workgroup partial reduced in index order by a one-workgroup kernel, or by
+// every workgroup of the kernel that needs it (alpha, where the partials are few).
+//
+// At 23k tets no kernel has work for the chip (184 workgroups of elements, 24 of
+// vertices at 256 each) and each is a chain of memory latencies, so the splits
+// below are made for many short chains. An iteration takes 42 us, 76 us before (launches included):
+// element product 23.7 -> 12.5 us (the update's loads no longer wait for its
+// stores, in workgroups of their own), vertex product 15.2 -> 7.6 us and a Chebyshev
+// step 6.6 -> 4.8 us (a lane to a component, 16 gathers in flight, 64 vertices a
+// workgroup), preconditioner 9.2 + 3.9 + 4.5 us -> 6.5 us in one launch. Sums keep
+// the order of one lane to a vertex and 256 vertices a workgroup: 500 iterations
+// amplify a last place to 1e-4 and, on some states, to the leading digits.
 #include <hip/hip_runtime.h>
 #include "device_math.h"
 #include "kernels.h"
@@ -41,7 +51,10 @@ namespace {
 constexpr int kTetBS = 128;
 constexpr int kVtxBS = 256;
 constexpr int kFinBS = 1024;
-constexpr int kGather = 8;  // indices / values in flight per gather batch
+constexpr int kLanes = 4;   // lanes of a vertex, one to a component (the fourth idles)
+constexpr int kSub = kVtxBS / kWave;  // workgroups of a vertex partial, see vertex_partial
+constexpr int kGather = 16;  // indices / values in flight per lane and gather batch
+constexpr int kUpdate = 4;   // entries of the p/x update per lane
 
 // Per-dimension element shape: corners, entries of s (Voigt, off-diagonals
 // weighted 2 by Sym), consistent-mass divisor (rho vol / 20 on a tet, / 12 on
@@ -68,15 +81,121 @@ __device__ __forceinline__ int xcd_index(int n) {
   return i < end ? (int)i : n;
 }
 
+// The same split with kLanes consecutive lanes to an item.
+__device__ __forceinline__ int xcd_row(int n) {
+  const int xcd = blockIdx.x & 7, lb = blockIdx.x >> 3;
+  const long long start = (long long)n * xcd / 8, end = (long long)n * (xcd + 1) / 8;
+  const long long i = start + (long long)lb * (blockDim.x / kLanes) + threadIdx.x / kLanes;
+  return i < end ? (int)i : n;
+}
+
+// y + the component r of a row's mass blocks times scale * src, in row order:
+// indices, then values, in flight together
+__device__ __forceinline__ double mass_gather(const int* __restrict__ col,
+                                              const double* __restrict__ mass, int b, int b1, int r,
+                                              const double* __restrict__ src, double scale) {
+  double y = 0;
+  for (; b < b1; b += kGather) {
+    int j[kGather];
+    double mm[kGather], w[kGather];
+#pragma unroll
+    for (int u = 0; u < kGather; ++u) {
+      j[u] = b + u < b1 ? col[b + u] : -1;
+      mm[u] = b + u < b1 ? mass[b + u] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kGather; ++u)
+      if (j[u] >= 0) w[u] = src[3 * j[u] + r];
+#pragma unroll
+    for (int u = 0; u < kGather; ++u)
+      if (j[u] >= 0) y += mm[u] * (w[u] * scale);
+  }
+  return y;
+}
+
+// The component r of the sum of the element contributions at a vertex, in order
+__device__ __forceinline__ double element_gather(const int* __restrict__ inc, int p, int p1, int r,
+                                                 const double* __restrict__ fe) {
+  double z = 0;
+  for (; p < p1; p += kGather) {
+    int ek[kGather];
+    double f[kGather];
+#pragma unroll
+    for (int u = 0; u < kGather; ++u) ek[u] = p + u < p1 ? inc[p + u] : -1;
+#pragma unroll
+    for (int u = 0; u < kGather; ++u)
+      if (ek[u] >= 0) f[u] = fe[(size_t)(ek[u] >> 2) * 12 + 3 * (ek[u] & 3) + r];
+#pragma unroll
+    for (int u = 0; u < kGather; ++u)
+      if (ek[u] >= 0) z += f[u];
+  }
+  return z;
+}
+
+// a . b over the components, which the first three lanes of the vertex hold
+__device__ __forceinline__ double dot3(double a, double b) {
+  const int l0 = (int)(threadIdx.x & (kWave - kLanes));
+  double d = 0;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) d += __shfl(a, l0 + r) * __shfl(b, l0 + r);
+  return d;
+}
+
+// Partial of a workgroup's 64 vertices (acc: the vertex's value in each of its
+// lanes). The kSub workgroups of 256 consecutive vertices lie side by side in
+// parts, and vertex_part adds them up: the order of one 256-lane workgroup.
+__device__ __forceinline__ void vertex_partial(double acc, double* parts) {
+  __shared__ double sm[kWave];
+  if ((threadIdx.x & (kLanes - 1)) == 0) sm[threadIdx.x / kLanes] = acc;
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  const double v = wave_sum(sm[threadIdx.x]);
+  const int xcd = blockIdx.x & 7, lb = blockIdx.x >> 3;
+  if (threadIdx.x == 0) parts[kSub * (8 * (lb / kSub) + xcd) + lb % kSub] = v;
+}
+// Partial i of ntet element workgroups followed by the vertex ones.
+__device__ __forceinline__ double mr_part(const double* __restrict__ parts, int ntet, int i) {
+  if (i < ntet) return parts[i];
+  const double* v = parts + ntet + kSub * (size_t)(i - ntet);
+  double r = v[0];
+#pragma unroll
+  for (int k = 1; k < kSub; ++k) r += v[k];
+  return r;
+}
+
 inline int blocks_for(int n, int bs) {
   if (n <= 0) return 0;
   const int per_xcd = (n + 7) / 8;
   return 8 * ((per_xcd + bs - 1) / bs);
 }
 
-// Sum of parts[0 .. n) in index order (strided by lane, then the block tree).
-__device__ __forceinline__ double fin_sum(const double* parts, int n, double* sm) {
-  return reduce_array<kFinBS, 0>(parts, n, 1, 0, sm);
+// Sum of ntet + nvtx partials in index order (strided by lane, then the block tree).
+__device__ __forceinline__ double fin_sum(const double* parts, int ntet, int nvtx, double* sm) {
+  double acc = 0;
+  for (int i = threadIdx.x; i < ntet + nvtx; i += kFinBS) acc += mr_part(parts, ntet, i);
+  return block_reduce_all<kFinBS, 0>(acc, sm);
+}
+// The same sum of at most kFinBS partials, to the last bit, by kTetBS threads.
+constexpr int kFoldParts = kFinBS;
+__device__ __forceinline__ double fold_sum(const double* parts, int ntet, int nvtx, double* sm) {
+  constexpr int kChunks = kFinBS / kTetBS;  // of kWave partials, per wave
+  const int n = ntet + nvtx, wid = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  double v[kChunks];
+#pragma unroll
+  for (int k = 0; k < kChunks; ++k) {
+    const int i = (wid + k * (kTetBS / kWave)) * kWave + lane;
+    v[k] = i < n ? mr_part(parts, ntet, i) : 0.0;
+  }
+#pragma unroll
+  for (int k = 0; k < kChunks; ++k)
+    if (k * kTetBS < n) {
+      v[k] = wave_sum(v[k]);
+      if (lane == 0) sm[wid + k * (kTetBS / kWave)] = v[k];
+    }
+  __syncthreads();
+  double r = sm[0];
+  for (int w = 1; w * kWave < n; ++w) r += sm[w];
+  return r;
 }
 
 // ---------------------------------------------------------------- setup
@@ -251,50 +370,17 @@ __global__ __launch_bounds__(kVtxBS) void k_kkt_rhs_vtx(int nfree, const int* __
                                                         const int* __restrict__ inc,
                                                         const double* __restrict__ fe, KktVec b,
                                                         double* __restrict__ parts) {
-  __shared__ double sm[kVtxBS / kWave];
-  const int i = xcd_index(nfree);
+  const int i = xcd_row(nfree), lane = threadIdx.x & (kLanes - 1), r = min(lane, 2);
   double acc = 0.0;
   if (i < nfree) {
-    double a[3] = {0, 0, 0};
-    const int p1 = inc_ptr[i + 1];
-    for (int p = inc_ptr[i]; p < p1; p += kGather) {  // batched gather, sums in order
-      int ek[kGather];
-      double f[kGather][3];
-#pragma unroll
-      for (int u = 0; u < kGather; ++u) ek[u] = p + u < p1 ? inc[p + u] : -1;
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (ek[u] >= 0) {
-          const double* src = fe + (size_t)(ek[u] >> 2) * 12 + 3 * (ek[u] & 3);
-#pragma unroll
-          for (int r = 0; r < 3; ++r) f[u][r] = src[r];
-        }
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (ek[u] >= 0)
-#pragma unroll
-          for (int r = 0; r < 3; ++r) a[r] += f[u][r];
-    }
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      b.x[3 * i + r] = a[r];
-      acc += a[r] * a[r];
-    }
+    const double a = element_gather(inc, inc_ptr[i], inc_ptr[i + 1], r, fe);
+    if (lane < 3) b.x[3 * i + r] = a;
+    acc = dot3(a, a);
   }
-  block_partial<kVtxBS, 0>(acc, parts, sm);
+  vertex_partial(acc, parts);
 }
 
 // ---------------------------------------------------------------- iteration
-// Update of the previous iteration, p_{k-1} = (w_{k-1} - r2 p_{k-2} -
-// r3 p_{k-3}) / r1 and x += beta_one c eta p_{k-1}, on one entry.
-__device__ __forceinline__ void pending_update(const MinresCtrl& c, long i, const double* wo,
-                                               const double* pa, const double* pb, double* pn,
-                                               double* x) {
-  const double p = (wo[i] / c.beta_prev - c.r2 * pa[i] - c.r3 * pb[i]) / c.r1;
-  pn[i] = p;
-  x[i] += c.coef * p;
-}
-
 struct MrVecs {
   KktVec wc;  // W_k (scale beta_k)
   KktVec vo;  // in: V_{k-1} (scale beta_{k-1}); out: V_{k+1} before alpha
@@ -305,38 +391,78 @@ struct MrVecs {
   KktVec x;   // solution
 };
 
+// Update of the previous iteration, p_{k-1} = (w_{k-1} - r2 p_{k-2} -
+// r3 p_{k-3}) / r1 and x += beta_one c eta p_{k-1}, by the workgroups of k_mr_tet
+// past those of the product (block = 0, 1, ... of them): the s part, the lambda
+// part, the x part. A streaming pass whose loads are all in flight before the
+// first store; inside the product it was a chain of 24 of them.
+inline __host__ __device__ int update_blocks(long n) {
+  return (int)((n + kUpdate * kTetBS - 1) / (kUpdate * kTetBS));
+}
+__device__ __forceinline__ void mr_update(const MinresCtrl& c, int block, long ne, long nx,
+                                          const MrVecs& V) {
+  const int be = update_blocks(ne);
+  const int part = block < be ? 0 : block < 2 * be ? 1 : 2;
+  const double* wo = part == 0 ? V.wo.s : part == 1 ? V.wo.l : V.wo.x;
+  const double* pa = part == 0 ? V.pa.s : part == 1 ? V.pa.l : V.pa.x;
+  const double* pb = part == 0 ? V.pb.s : part == 1 ? V.pb.l : V.pb.x;
+  double* pn = part == 0 ? V.pn.s : part == 1 ? V.pn.l : V.pn.x;
+  double* x = part == 0 ? V.x.s : part == 1 ? V.x.l : V.x.x;
+  const long n = part == 2 ? nx : ne;
+  const long i0 = (long)(block - part * be) * kUpdate * kTetBS + threadIdx.x;
+  double w[kUpdate], a[kUpdate], b[kUpdate], xv[kUpdate];
+#pragma unroll
+  for (int u = 0; u < kUpdate; ++u) {
+    const long i = i0 + u * kTetBS;
+    if (i < n) {
+      w[u] = wo[i];
+      a[u] = pa[i];
+      b[u] = pb[i];
+      xv[u] = x[i];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kUpdate; ++u) {
+    const long i = i0 + u * kTetBS;
+    if (i < n) {
+      const double p = (w[u] / c.beta_prev - c.r2 * a[u] - c.r3 * b[u]) / c.r1;
+      pn[i] = p;
+      x[i] = xv[u] + c.coef * p;
+    }
+  }
+}
+
 template <typename Real, int DIM>
 __global__ __launch_bounds__(kTetBS) void k_mr_tet(TetMeshDev m, const MinresCtrl* __restrict__ ctrl,
                                                    const Real* __restrict__ dsdF,
                                                    const Real* __restrict__ Hpsi, MrVecs V,
                                                    double* __restrict__ fe,
-                                                   double* __restrict__ parts) {
+                                                   double* __restrict__ parts, int nproduct) {
   using E = Elem<DIM>;
   constexpr int NC = E::NC, NS = E::NS, NF = E::NF;
   constexpr int kFePitch = 13;  // x-row contributions staged per tet (odd pitch: LDS banks)
   __shared__ double sm[kTetBS / kWave];
   __shared__ double fe_stage[kTetBS * kFePitch];
   const MinresCtrl c = *ctrl;
-  const int e = xcd_index(m.nT);
   const int nT = m.nT;
-  if (c.pending && e < nT) {
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      pending_update(c, (long)i * nT + e, V.wo.s, V.pa.s, V.pb.s, V.pn.s, V.x.s);
-      pending_update(c, (long)i * nT + e, V.wo.l, V.pa.l, V.pb.l, V.pn.l, V.x.l);
-    }
+  if ((int)blockIdx.x >= nproduct) {
+    if (c.pending) mr_update(c, (int)blockIdx.x - nproduct, (long)NS * nT, 3L * m.nfree, V);
+    return;
   }
+  const int e = xcd_index(m.nT);
   if (c.done) return;
   double acc = 0.0;
   if (e < nT) {
     const double vol = m.vol[e];
     const double ib = 1.0 / c.beta;
     const double ratio = c.beta / c.beta_prev;
-    double ws[NS], wl[NS];
+    double ws[NS], wl[NS], vo_s[NS], vo_l[NS];
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
       ws[i] = V.wc.s[i * nT + e] * ib;
       wl[i] = V.wc.l[i * nT + e] * ib;
+      vo_s[i] = V.vo.s[i * nT + e];
+      vo_l[i] = V.vo.l[i * nT + e];
     }
     // Jloc w_x over the free corners
     const int4 t = m.T[e];
@@ -394,11 +520,11 @@ __global__ __launch_bounds__(kTetBS) void k_mr_tet(TetMeshDev m, const MinresCtr
       const double yl = vol * E::symw(i) * (ws[i] - u[i]);
       const long is = (long)i * nT + e;
       // v_new = K w - beta v_old, v_old = V_{k-1} / beta_{k-1}
-      const double vs = ys - ratio * V.vo.s[is];
-      const double vl = yl - ratio * V.vo.l[is];
+      const double vs = ys - ratio * vo_s[i];
+      const double vl = yl - ratio * vo_l[i];
       V.vo.s[is] = vs;
       V.vo.l[is] = vl;
-      acc += vs * ws[i] + vl * wl[i];
+      acc += fma(vs, ws[i], vl * wl[i]);
     }
   }
   // the staged x-row contributions of this wave's live tets, which are a
@@ -425,115 +551,124 @@ __global__ __launch_bounds__(kVtxBS) void k_mr_vertex(int nfree, const int* __re
                                                       const double* __restrict__ fe,
                                                       const MinresCtrl* __restrict__ ctrl, MrVecs V,
                                                       double* __restrict__ parts) {
-  __shared__ double sm[kVtxBS / kWave];
   const MinresCtrl c = *ctrl;
-  const int i = xcd_index(nfree);
-  if (c.pending && i < nfree) {
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-      pending_update(c, 3L * i + r, V.wo.x, V.pa.x, V.pb.x, V.pn.x, V.x.x);
-  }
   if (c.done) return;
+  const int i = xcd_row(nfree), lane = threadIdx.x & (kLanes - 1), r = min(lane, 2);
   double acc = 0.0;
   if (i < nfree) {
     const double ib = 1.0 / c.beta;
     const double ratio = c.beta / c.beta_prev;
-    // both gathers in batches of kGather: indices, then values, in flight
-    // together (the sums keep their order)
-    double y[3] = {0, 0, 0};
-    const int b1 = rowptr[i + 1];
-    for (int b = rowptr[i]; b < b1; b += kGather) {
-      int j[kGather];
-      double mm[kGather], w[kGather][3];
-#pragma unroll
-      for (int u = 0; u < kGather; ++u) {
-        j[u] = b + u < b1 ? col[b + u] : -1;
-        mm[u] = b + u < b1 ? mass[b + u] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (j[u] >= 0)
-#pragma unroll
-          for (int r = 0; r < 3; ++r) w[u][r] = V.wc.x[3 * j[u] + r];
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (j[u] >= 0)
-#pragma unroll
-          for (int r = 0; r < 3; ++r) y[r] += mm[u] * (w[u][r] * ib);
-    }
-    double z[3] = {0, 0, 0};
-    const int p1 = inc_ptr[i + 1];
-    for (int p = inc_ptr[i]; p < p1; p += kGather) {
-      int ek[kGather];
-      double f[kGather][3];
-#pragma unroll
-      for (int u = 0; u < kGather; ++u) ek[u] = p + u < p1 ? inc[p + u] : -1;
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (ek[u] >= 0) {
-          const double* src = fe + (size_t)(ek[u] >> 2) * 12 + 3 * (ek[u] & 3);
-#pragma unroll
-          for (int r = 0; r < 3; ++r) f[u][r] = src[r];
-        }
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (ek[u] >= 0)
-#pragma unroll
-          for (int r = 0; r < 3; ++r) z[r] += f[u][r];
-    }
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      const long ir = 3L * i + r;
-      const double vn = (y[r] + z[r]) - ratio * V.vo.x[ir];
-      V.vo.x[ir] = vn;
-      acc += vn * (V.wc.x[ir] * ib);
-    }
+    const long ir = 3L * i + r;
+    const double vo = V.vo.x[ir], wi = V.wc.x[ir];
+    const double y = mass_gather(col, mass, rowptr[i], rowptr[i + 1], r, V.wc.x, ib);
+    const double z = element_gather(inc, inc_ptr[i], inc_ptr[i + 1], r, fe);
+    const double vn = (y + z) - ratio * vo;
+    if (lane < 3) V.vo.x[ir] = vn;
+    acc = dot3(vn, wi * ib);
   }
-  block_partial<kVtxBS, 0>(acc, parts, sm);
+  vertex_partial(acc, parts);
 }
 
 // alpha = v_new . w; the pending update has been applied by now.
 __global__ __launch_bounds__(kFinBS) void k_mr_fin_alpha(MinresCtrl* ctrl, const double* parts,
-                                                         int nparts) {
+                                                         int ntet, int nvtx) {
   __shared__ double sm[kFinBS / kWave];
   const bool done = ctrl->done;
   __syncthreads();
   if (threadIdx.x == 0) ctrl->pending = 0;
   if (done) return;
-  const double a = fin_sum(parts, nparts, sm);
+  const double a = fin_sum(parts, ntet, nvtx, sm);
   if (threadIdx.x == 0) ctrl->alpha = a;
 }
 
-// v_new -= alpha v_k (init: alpha = 0, v_k absent); w_new = P v_new on the
-// element parts: Hloc^-1 = Hpsi^-1 / vol on s, S_e^-1 on lambda.
+// v_new -= alpha v_k (init: alpha = 0, v_k absent) and w_new = P v_new: by the
+// first nelem workgroups on the element parts, Hloc^-1 = Hpsi^-1 / vol on s and
+// S_e^-1 on lambda; by the others on the x part, with the first Chebyshev step of
+// the mass block, r = v_new, d = D^-1 r / theta, z = d. With nvtx > 0 every
+// workgroup sums alpha from parts_a itself while its loads are in flight
+// (k_mr_fin_alpha and its launch took 6 us an iteration), and the first stores it.
 template <typename Real, int DIM>
-__global__ __launch_bounds__(kTetBS) void k_mr_prec_tet(TetMeshDev m, const MinresCtrl* __restrict__ ctrl,
-                                                        int init, const Real* __restrict__ Hinv,
-                                                        const double* __restrict__ Sinv, KktVec vn,
-                                                        KktVec vc, KktVec wn,
-                                                        double* __restrict__ parts) {
+__global__ __launch_bounds__(kTetBS) void k_mr_prec(TetMeshDev m, MinresCtrl* ctrl, int init,
+                                                    int nelem, int nvtx,
+                                                    const double* __restrict__ parts_a,
+                                                    const Real* __restrict__ Hinv,
+                                                    const double* __restrict__ Sinv,
+                                                    const double* __restrict__ dinv, double theta,
+                                                    KktVec vn, KktVec vc, KktVec wn,
+                                                    double* __restrict__ cr,
+                                                    double* __restrict__ cd,
+                                                    double* __restrict__ parts) {
   using E = Elem<DIM>;
-  constexpr int NS = E::NS;
-  __shared__ double sm[kTetBS / kWave];
-  const MinresCtrl c = *ctrl;
-  if (!init && c.done) return;
+  constexpr int NS = E::NS, NH = NS * (NS + 1) / 2;
+  __shared__ double sm[kFinBS / kWave];
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (!init && ctrl->done) {
+    if (nvtx > 0 && first) ctrl->pending = 0;
+    return;
+  }
+  const double beta = ctrl->beta;
+  auto combine = [&] {  // alpha / beta; every thread comes here
+    if (init) return 0.0;
+    if (nvtx == 0) return ctrl->alpha / beta;
+    const double alpha = fold_sum(parts_a, nelem, nvtx, sm);
+    if (first) {
+      ctrl->alpha = alpha;
+      ctrl->pending = 0;  // the update of the previous iteration has been applied
+    }
+    return alpha / beta;
+  };
+  if ((int)blockIdx.x >= nelem) {
+    const long n = 3L * m.nfree;
+    const long ir = (long)((int)blockIdx.x - nelem) * kTetBS + threadIdx.x;
+    double v = 0, c = 0, di = 0;
+    if (ir < n) {
+      v = vn.x[ir];
+      if (!init) c = vc.x[ir];
+      di = dinv[ir / 3];
+    }
+    const double ab = combine();
+    if (ir >= n) return;
+    if (!init) {
+      v -= ab * c;
+      vn.x[ir] = v;
+    }
+    const double d = di * v / theta;
+    cr[ir] = v;
+    cd[ir] = d;
+    wn.x[ir] = d;
+    return;
+  }
   const int e = xcd_index(m.nT);
   const int nT = m.nT;
-  double acc = 0.0;
+  double vs[NS], vl[NS], cs[NS], cl[NS], hi[NH], si[NH], vol = 1.0;
   if (e < nT) {
-    const double ab = init ? 0.0 : c.alpha / c.beta;
-    const double vol = m.vol[e];
-    double vs[NS], vl[NS];
+    vol = m.vol[e];
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
       const long is = (long)i * nT + e;
-      vs[i] = init ? vn.s[is] : vn.s[is] - ab * vc.s[is];
-      vl[i] = init ? vn.l[is] : vn.l[is] - ab * vc.l[is];
-      if (!init) {
+      vs[i] = vn.s[is];
+      vl[i] = vn.l[is];
+      cs[i] = init ? 0.0 : vc.s[is];
+      cl[i] = init ? 0.0 : vc.l[is];
+    }
+#pragma unroll
+    for (int k = 0; k < NH; ++k) {
+      hi[k] = (double)Hinv[k * nT + e];
+      si[k] = Sinv[k * nT + e];
+    }
+  }
+  const double ab = combine();
+  double acc = 0.0;
+  if (e < nT) {
+    if (!init)
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        const long is = (long)i * nT + e;
+        vs[i] -= ab * cs[i];
+        vl[i] -= ab * cl[i];
         vn.s[is] = vs[i];
         vn.l[is] = vl[i];
       }
-    }
     const double iv = 1.0 / vol;
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
@@ -541,8 +676,8 @@ __global__ __launch_bounds__(kTetBS) void k_mr_prec_tet(TetMeshDev m, const Minr
 #pragma unroll
       for (int j = 0; j < NS; ++j) {
         const int k = E::sym(i, j);
-        a += (double)Hinv[k * nT + e] * vs[j];
-        b += Sinv[k * nT + e] * vl[j];
+        a += hi[k] * vs[j];
+        b += si[k] * vl[j];
       }
       const long is = (long)i * nT + e;
       const double zs = a * iv;
@@ -552,34 +687,6 @@ __global__ __launch_bounds__(kTetBS) void k_mr_prec_tet(TetMeshDev m, const Minr
     }
   }
   block_partial<kTetBS, 0>(acc, parts, sm);
-}
-
-// x part: v_new -= alpha v_k, then the first Chebyshev step of the mass block:
-// r = v_new, d = D^-1 r / theta, z = d.
-__global__ __launch_bounds__(kVtxBS) void k_mr_prec_vtx0(int nfree, const MinresCtrl* __restrict__ ctrl,
-                                                         int init, const double* __restrict__ dinv,
-                                                         double theta, KktVec vn, KktVec vc,
-                                                         KktVec wn, double* __restrict__ cr,
-                                                         double* __restrict__ cd) {
-  const MinresCtrl c = *ctrl;
-  if (!init && c.done) return;
-  const int i = xcd_index(nfree);
-  if (i >= nfree) return;
-  const double ab = init ? 0.0 : c.alpha / c.beta;
-  const double di = dinv[i];
-#pragma unroll
-  for (int r = 0; r < 3; ++r) {
-    const long ir = 3L * i + r;
-    double v = vn.x[ir];
-    if (!init) {
-      v -= ab * vc.x[ir];
-      vn.x[ir] = v;
-    }
-    const double d = di * v / theta;
-    cr[ir] = v;
-    cd[ir] = d;
-    wn.x[ir] = d;
-  }
 }
 
 // One Chebyshev step: r -= PMP d_in; d_out = c1 d_in + c2 D^-1 r; z += d_out.
@@ -594,54 +701,32 @@ __global__ __launch_bounds__(kVtxBS) void k_mr_cheb(int nfree, const int* __rest
                                                     double* __restrict__ cr, KktVec vn, KktVec wn,
                                                     int last, int init,
                                                     double* __restrict__ parts) {
-  __shared__ double sm[kVtxBS / kWave];
   if (!init && ctrl->done) return;
-  const int i = xcd_index(nfree);
+  const int i = xcd_row(nfree), lane = threadIdx.x & (kLanes - 1), r = min(lane, 2);
   double acc = 0.0;
   if (i < nfree) {
-    double y[3] = {0, 0, 0};
-    const int b1 = rowptr[i + 1];
-    for (int b = rowptr[i]; b < b1; b += kGather) {  // batched gather, sums in order
-      int j[kGather];
-      double mm[kGather], w[kGather][3];
-#pragma unroll
-      for (int u = 0; u < kGather; ++u) {
-        j[u] = b + u < b1 ? col[b + u] : -1;
-        mm[u] = b + u < b1 ? mass[b + u] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (j[u] >= 0)
-#pragma unroll
-          for (int r = 0; r < 3; ++r) w[u][r] = d_in[3 * j[u] + r];
-#pragma unroll
-      for (int u = 0; u < kGather; ++u)
-        if (j[u] >= 0)
-#pragma unroll
-          for (int r = 0; r < 3; ++r) y[r] += mm[u] * w[u][r];
-    }
-    const double di = dinv[i];
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      const long ir = 3L * i + r;
-      const double rr = cr[ir] - y[r];
+    const long ir = 3L * i + r;
+    const double di = dinv[i], ri = cr[ir], dr = d_in[ir], zr = wn.x[ir], vr = vn.x[ir];
+    const double y = mass_gather(col, mass, rowptr[i], rowptr[i + 1], r, d_in, 1.0);
+    const double rr = ri - y;
+    const double d = fma(c2 * di, rr, c1 * dr);
+    const double z = zr + d;
+    if (lane < 3) {
       cr[ir] = rr;
-      const double d = c1 * d_in[ir] + c2 * di * rr;
       d_out[ir] = d;
-      const double z = wn.x[ir] + d;
       wn.x[ir] = z;
-      acc += vn.x[ir] * z;
     }
+    if (last) acc = dot3(vr, z);
   }
-  if (last) block_partial<kVtxBS, 0>(acc, parts, sm);
+  if (last) vertex_partial(acc, parts);
 }
 
 // beta_new, the Givens rotation and the stopping test of one iteration.
 __global__ __launch_bounds__(kFinBS) void k_mr_fin_beta(MinresCtrl* ctrl, const double* parts,
-                                                        int nparts) {
+                                                        int ntet, int nvtx) {
   __shared__ double sm[kFinBS / kWave];
   if (ctrl->done) return;
-  const double b2 = fin_sum(parts, nparts, sm);
+  const double b2 = fin_sum(parts, ntet, nvtx, sm);
   if (threadIdx.x != 0) return;
   MinresCtrl c = *ctrl;
   if (!(b2 >= 0.0)) {  // preconditioner not positive definite (or NaN)
@@ -687,11 +772,11 @@ __global__ void k_mr_ctrl_unit(MinresCtrl* ctrl) {
 
 // Scalars after the right-hand side and its preconditioned image.
 __global__ __launch_bounds__(kFinBS) void k_mr_fin_init(MinresCtrl* ctrl, const double* parts_b,
-                                                        const double* parts_w, int nparts,
+                                                        const double* parts_w, int ntet, int nvtx,
                                                         double tol, int max_iters) {
   __shared__ double sm[kFinBS / kWave];
-  const double rhs2 = fin_sum(parts_b, nparts, sm);
-  const double b2 = fin_sum(parts_w, nparts, sm);
+  const double rhs2 = fin_sum(parts_b, ntet, nvtx, sm);
+  const double b2 = fin_sum(parts_w, ntet, nvtx, sm);
   if (threadIdx.x != 0) return;
   MinresCtrl c{};
   c.rhs2 = rhs2;
@@ -719,7 +804,7 @@ __global__ __launch_bounds__(kFinBS) void k_mr_fin_init(MinresCtrl* ctrl, const 
 }  // namespace
 
 int kkt_tet_blocks(int nT) { return blocks_for(nT, kTetBS); }
-int kkt_vertex_blocks(int nfree) { return blocks_for(nfree, kVtxBS); }
+int kkt_vertex_blocks(int nfree) { return kSub * blocks_for(nfree, kVtxBS); }
 
 template <typename Real>
 void launch_kkt_setup(const KktSystem<Real>& S, hipStream_t st) {
@@ -742,16 +827,18 @@ template <typename Real>
 void launch_precondition(const KktSystem<Real>& S, int init, KktVec vn, KktVec vc, KktVec wn,
                          hipStream_t st) {
   const int nbT = kkt_tet_blocks(S.m.nT), nbV = kkt_vertex_blocks(S.m.nfree);
-  if (nbT > 0)
-    if (S.m.dim == 2)
-      hipLaunchKernelGGL((k_mr_prec_tet<Real, 2>), dim3(nbT), dim3(kTetBS), 0, st, S.m, S.ctrl,
-                         init, S.Hinv, S.Sinv, vn, vc, wn, S.parts[1]);
-    else
-      hipLaunchKernelGGL((k_mr_prec_tet<Real, 3>), dim3(nbT), dim3(kTetBS), 0, st, S.m, S.ctrl,
-                         init, S.Hinv, S.Sinv, vn, vc, wn, S.parts[1]);
+  const int nvtx = nbV / kSub;
+  const bool fold = !init && nvtx > 0 && nbT + nvtx <= kFoldParts;
+  if (!init && !fold)
+    hipLaunchKernelGGL(k_mr_fin_alpha, dim3(1), dim3(kFinBS), 0, st, S.ctrl, S.parts[0], nbT,
+                       nvtx);
+  const dim3 grid(nbT + (int)((3L * S.m.nfree + kTetBS - 1) / kTetBS));
+  if (grid.x == 0) return;
+  auto kernel = S.m.dim == 2 ? k_mr_prec<Real, 2> : k_mr_prec<Real, 3>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kTetBS), 0, st, S.m, S.ctrl, init, nbT, fold ? nvtx : 0, S.parts[0],
+                     S.Hinv, S.Sinv, S.mdinv, kChebTheta, vn, vc, wn, S.cheb_r, S.cheb_d[0],
+                     S.parts[1]);
   if (nbV == 0) return;
-  hipLaunchKernelGGL(k_mr_prec_vtx0, dim3(nbV), dim3(kVtxBS), 0, st, S.m.nfree, S.ctrl, init,
-                     S.mdinv, kChebTheta, vn, vc, wn, S.cheb_r, S.cheb_d[0]);
   const double sigma = kChebTheta / kChebDelta;
   double rho = 1.0 / sigma;
   for (int j = 1; j < kMassChebSteps; ++j) {
@@ -763,6 +850,19 @@ void launch_precondition(const KktSystem<Real>& S, int init, KktVec vn, KktVec v
                        S.parts[1] + nbT);
     rho = rho1;
   }
+}
+
+// The element part of v_new = K w - beta v_old, with the pending p/x update.
+template <typename Real>
+void launch_element_product(const KktSystem<Real>& S, const MrVecs& V, bool update,
+                            hipStream_t st) {
+  const int nbT = kkt_tet_blocks(S.m.nT), ns = S.m.dim == 2 ? 3 : 6;
+  int grid = nbT;
+  if (update) grid += 2 * update_blocks((long)ns * S.m.nT) + update_blocks(3L * S.m.nfree);
+  if (grid == 0) return;
+  auto kernel = S.m.dim == 2 ? k_mr_tet<Real, 2> : k_mr_tet<Real, 3>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kTetBS), 0, st, S.m, S.ctrl, S.dsdF, S.Hpsi, V, S.fe,
+                     S.parts[0], nbT);
 }
 }  // namespace
 
@@ -783,7 +883,7 @@ void launch_minres_init(const KktSystem<Real>& S, const double* x_full, const In
                        S.inc, S.fe, b, S.parts[0] + nbT);
   launch_precondition(S, 1, b, b, w, st);
   hipLaunchKernelGGL(k_mr_fin_init, dim3(1), dim3(kFinBS), 0, st, S.ctrl, S.parts[0],
-                     S.parts[1], nbT + nbV, tol, max_iters);
+                     S.parts[1], nbT, nbV / kSub, tol, max_iters);
 }
 
 template <typename Real>
@@ -800,21 +900,15 @@ void launch_minres_iteration(const KktSystem<Real>& S, const MinresBuffers& B, l
   V.pn = B.p[mod3(k - 1)];  // p_{k-1} replaces p_{k-4}
   V.x = B.x;
   if (tet_ev) (void)hipEventRecord(tet_ev[0], st);
-  if (nbT > 0)
-    if (S.m.dim == 2)
-      hipLaunchKernelGGL((k_mr_tet<Real, 2>), dim3(nbT), dim3(kTetBS), 0, st, S.m, S.ctrl, S.dsdF,
-                         S.Hpsi, V, S.fe, S.parts[0]);
-    else
-      hipLaunchKernelGGL((k_mr_tet<Real, 3>), dim3(nbT), dim3(kTetBS), 0, st, S.m, S.ctrl, S.dsdF,
-                         S.Hpsi, V, S.fe, S.parts[0]);
+  launch_element_product(S, V, true, st);
   if (tet_ev) (void)hipEventRecord(tet_ev[1], st);
   if (nbV > 0)
     hipLaunchKernelGGL(k_mr_vertex, dim3(nbV), dim3(kVtxBS), 0, st, S.m.nfree, S.rowptr, S.col,
                        S.mass, S.inc_ptr, S.inc, S.fe, S.ctrl, V, S.parts[0] + nbT);
-  hipLaunchKernelGGL(k_mr_fin_alpha, dim3(1), dim3(kFinBS), 0, st, S.ctrl, S.parts[0], nbT + nbV);
   // v_new (in V_{k-1}'s buffer) -= alpha v_k; w_new into W_{k-1}'s buffer
   launch_precondition(S, 0, B.v[(k + 1) & 1], B.v[k & 1], B.w[(k + 1) & 1], st);
-  hipLaunchKernelGGL(k_mr_fin_beta, dim3(1), dim3(kFinBS), 0, st, S.ctrl, S.parts[1], nbT + nbV);
+  hipLaunchKernelGGL(k_mr_fin_beta, dim3(1), dim3(kFinBS), 0, st, S.ctrl, S.parts[1], nbT,
+                     nbV / kSub);
 }
 
 template <typename Real>
@@ -836,13 +930,7 @@ void launch_kkt_apply(const KktSystem<Real>& S, int which, KktVec in, KktVec out
   V.wo = in;
   V.vo = out;
   V.pa = V.pb = V.pn = V.x = scratch;
-  if (nbT > 0)
-    if (S.m.dim == 2)
-      hipLaunchKernelGGL((k_mr_tet<Real, 2>), dim3(nbT), dim3(kTetBS), 0, st, S.m, S.ctrl, S.dsdF,
-                         S.Hpsi, V, S.fe, S.parts[0]);
-    else
-      hipLaunchKernelGGL((k_mr_tet<Real, 3>), dim3(nbT), dim3(kTetBS), 0, st, S.m, S.ctrl, S.dsdF,
-                         S.Hpsi, V, S.fe, S.parts[0]);
+  launch_element_product(S, V, false, st);
   if (nbV > 0)
     hipLaunchKernelGGL(k_mr_vertex, dim3(nbV), dim3(kVtxBS), 0, st, S.m.nfree, S.rowptr, S.col,
                        S.mass, S.inc_ptr, S.inc, S.fe, S.ctrl, V, S.parts[0] + nbT);

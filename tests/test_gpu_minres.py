@@ -228,3 +228,22 @@ def test_minres_2d_timesteps_match_oracle(native, oracle, precision, tol):
         disp = np.abs(ref.positions() - sc.V[:, :2]).max()
         assert disp > 1e-4
         assert np.abs(dev.positions()[:, :2] - ref.positions()).max() < tol * disp
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(5, 3, 3), (50, 17, 17), (60, 19, 19)])
+def test_minres_alpha_sum_on_both_sides_of_its_line(native, oracle, nx, ny, nz):
+    """alpha is summed inside the preconditioner kernel up to 1024 partials
+    (270 tets: 1 chunk of 64; 87k tets: 12), by a kernel of its own above (130k).
+    Four iterations against the oracle: each sum of n = 3e5..1e6 terms rounds to
+    sqrt(n) 1e-16 < 1e-12 of its terms' size, and few iterations amplify that by
+    less than the 1e3 left to the bar."""
+    sc = scenes.beam_scene(nx, ny, nz, seed=4, mixed=True, solver=SOLVER, max_newton=1,
+                           itr_tol=1e-300, max_iters=4)
+    print(f"minres alpha: nT={sc.nT}", flush=True)
+    dev = native.Sim(sc, precision="fp64")
+    ref = oracle.Sim(sc)
+    for sim in (dev, ref):
+        sim.update_system()
+        sim.solve()
+    for name in ("dx", "ds", "lambda"):
+        assert relerr(dev.get(name), ref.get(name)) < 1e-9, name
