@@ -178,12 +178,13 @@ int mfem_sim_spmv_tuning(mfem_sim* sim, double* times, int* count, int* chosen, 
  * configures it). Force shape `variant` (0-7: lanes per block row, blocks
  * in flight per lane and workgroup size as listed in k_solver.hip) on a grid
  * of `blocks` workgroups (a multiple of 8 in [8, 4096], or 0 for the
- * default); variant -1 restores autotuning on the next solve. */
+ * default); variant -1 restores the default: the resident kernel where the
+ * system fits the chip, else autotuning on the next solve. */
 int mfem_sim_set_cg_shape(mfem_sim* sim, int variant, int blocks);
 /* CG kernel autotuner result: every (shape, grid) pair timed on the first
  * solve (times[count] ms per iteration, variants[count], grids[count]; pass
  * NULL arrays to query count), the index of the chosen pair (-1 when untuned
- * or forced), and the chosen lanes-per-row / blocks in flight per lane /
+ * or forced; count is 0 where the resident kernel solves), and the chosen lanes-per-row / blocks in flight per lane /
  * workgroup size / grid. */
 int mfem_sim_cg_tuning(mfem_sim* sim, double* times, int* variants, int* grids, int* count,
                        int* chosen, int* lanes, int* unroll, int* threads, int* blocks);
@@ -227,7 +228,8 @@ int mfem_batch_cg_shape(mfem_batch* batch, int* variant, int* rows_per_workgroup
 /* hipGraph replay of the batch's Newton phases (no counterpart in the
  * reference; off by default): with on = 1 the element update + assembly phase of every
  * Newton iteration is one captured graph from the second step on, and CG
- * iterations are replayed in captured groups of 16; on = 0 launches every
+ * iterations, where they are launches of their own (a forced shape, or beams that
+ * the resident CG does not take), are replayed in captured groups of 16; on = 0 launches every
  * kernel separately. Results are identical bit for bit. */
 int mfem_batch_set_graphs(mfem_batch* batch, int on);
 /* Host submissions since creation: of the update + assembly phase, of the CG
