@@ -81,11 +81,7 @@ def run_gpu(scene, precision, steps, warmup, profile=True, element_kernel=0):
         sim.set_element_kernel(element_kernel)
     for _ in range(warmup):
         sim.step()
-    if profile:
-        sim.set_profiling(1)
     newton = pcg = 0
-    spmv_ms = 0.0
-    spmv_n = 0
     t0 = time.perf_counter()
     per_step = []
     ls_fail = []
@@ -111,17 +107,25 @@ def run_gpu(scene, precision, steps, warmup, profile=True, element_kernel=0):
               f"ls failures {st['ls_fail']}", file=sys.stderr, flush=True)
         newton += st["newton_iters"]
         pcg += st["pcg_iters"]
-        spmv_ms += st["spmv_ms"]
-        spmv_n += st["spmv_count"]
     elapsed = time.perf_counter() - t0
     nfree, nnzb, vb = sim.matrix_info()
     x = sim.positions()
     # per-phase device times (update, solve, line search) from one more,
     # untimed timestep with the phase events on: each event is a marker in
     # the stream that costs the device a few microseconds
-    sim.set_profiling(3 if profile else 2)
+    sim.set_profiling(2)
     sim.step()
     st = sim.stats()
+    # the iteration kernels' own times from two further untimed timesteps: the
+    # bandwidth profiling launches every CG iteration by itself (the first of
+    # them times the kernel shapes)
+    spmv_ms, spmv_n = 0.0, 0
+    if profile:
+        sim.set_profiling(1)
+        sim.step()
+        sim.step()
+        prof = sim.stats()
+        spmv_ms, spmv_n = prof["spmv_ms"], prof["spmv_count"]
     tuning = None
     if scene.solver == "eigen-pcg-diag":
         trials, chosen, shape = sim.cg_tuning()
@@ -582,7 +586,10 @@ def main():
                                "5 dot-product partials)",
                      "bytes_per_launch": bytes_spmv, "avg_launch_ms": avg_spmv_ms,
                      "launches": mixed["spmv_n"],
-                     "timing": "per-workgroup device wall-clock stamps, span of each launch"},
+                     "timing": "per-workgroup device wall-clock stamps, span of each launch, in an "
+                               "untimed timestep that launches every iteration by itself; the "
+                               "timed ones solve in one launch where the system fits the chip"},
+        "cg_us_per_iteration": 1e3 * mixed["last"]["solve_ms"] / max(mixed["last"]["pcg_iters"], 1),
         "cpu_baseline": cpu,
         "phase_ms_untimed_step": {k: mixed["last"][k] for k in ("update_ms", "solve_ms", "ls_ms")},
         "cg_autotune": mixed["tuning"],
