@@ -340,7 +340,7 @@ bool BatchSim::run_cg_resident(const double* b, double* x, const std::vector<dou
   res_q_.resize(9 * (size_t)m.nfree(), sizeof(T) == 4);
   res_parts_.resize(48 * (size_t)kCgResidentMaxWg);
   res_spill_.resize(res_spill_n_, sizeof(T) == 4);
-  res_flag_.resize(1);
+  res_flag_.resize(1 + (size_t)nsim_);
   MFEM_HIP_CHECK(hipMemcpyAsync(res_sys_.data(), hs, sizeof(CgResidentSys) * n,
                                 hipMemcpyHostToDevice, st));
   MFEM_HIP_CHECK(hipMemcpyAsync(res_team_.data(), ht, sizeof(int) * t, hipMemcpyHostToDevice, st));
@@ -355,6 +355,7 @@ bool BatchSim::run_cg_resident(const double* b, double* x, const std::vector<dou
   A.q = reinterpret_cast<decltype(A.q)>(res_q_.template as<T>());
   A.parts = res_parts_.data();
   A.spill = res_spill_.template as<T>();
+  A.nsys = nsim_;
   A.flag = res_flag_.data();
   A.ctrl = ctrls_.data();
   A.mirror = pinned_ctrl_->device<PcgCtrl>();

@@ -592,7 +592,7 @@ bool PcgSolver<DIM>::run_cg_resident(const double* b, double* x, double tol, int
   res_q_.resize(9 * (size_t)m.nfree(), sizeof(T) == 4);
   res_spill_.resize(plan.spill, sizeof(T) == 4);
   res_parts_.resize(24 * (size_t)kCgResidentMaxWg);
-  res_flag_.resize(1);
+  res_flag_.resize(2);
   CgResidentArgs<T> A;
   A.nrows = m.nfree();
   A.rowptr = m.d_rowptr.data();

@@ -376,7 +376,7 @@ class PcgSolver : public LinearSolver<DIM> {
   RealArray res_q_;              // resident CG: exchange words of q, 3 slots
   DeviceArray<unsigned long long> res_parts_;  // resident CG: exchanged partial sums
   RealArray res_spill_;          // resident CG: block values beyond registers and LDS
-  DeviceArray<int> res_flag_;    // resident CG: a workgroup gave up
+  DeviceArray<int> res_flag_;    // resident CG: a workgroup gave up; the verdict
   mfemhip::PcgCtrl last_{};      // control block at the end of the last CG solve
   std::unique_ptr<PinnedBuffer> pinned_;  // mapped host copy of the control block
   double wall_khz_ = 100000.0;   // device wall-clock rate

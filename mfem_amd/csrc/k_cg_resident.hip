@@ -41,6 +41,18 @@
 // a wait that lasts longer than `wait_ticks` of the wall clock raises a flag
 // that every other wait polls; all workgroups then leave, the control block
 // says so, and the host solves with the one-kernel-per-iteration CG instead.
+//
+// Verdict. A solve has one verdict word, which leaves 0 once, by compare-exchange:
+// workgroup 0 makes it `done` when it has the sums that stop the solve, and a
+// workgroup that gives up a wait makes it `expired`. Whoever loses follows the
+// winner, so all workgroups leave a solve with the same answer:
+//   - a workgroup whose wait runs out behind `done` keeps polling. Workgroup 0 has
+//     seen the sums of every workgroup, so each of them is past every other wait
+//     of this solve, and the sums that it still polls are all there;
+//   - a workgroup that has the stopping sums itself waits for the verdict before
+//     it writes its rows of x. The sums are published, so workgroup 0 gets them
+//     too, or leaves by a wait that ran out, and gives the verdict either way.
+// x is therefore written whole, or not at all.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cfloat>
@@ -154,20 +166,33 @@ __device__ __forceinline__ void publish_stop(const PcgCtrl& c, PcgCtrl* ctrl, Pc
 // v, the same in every lane, as one scalar
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Flag word of a solve: 0 while it runs, 1 after a wait expired.
+// Makes the verdict v if there is none yet; returns the verdict.
+__device__ __forceinline__ int decide(int* verdict, int v) {
+  int is = 0;
+  return __hip_atomic_compare_exchange_strong(verdict, &is, v, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT)
+             ? v
+             : is;
+}
+
+// Bounded wait. The flag is 0 until a workgroup of the launch gives up.
 struct Waiter {
   int* flag;
+  int* verdict;
   long long ticks;
   long long start = 0;
   int polls = 0;
   // true when the wait has to be given up
   __device__ __forceinline__ bool expired() {
     if (++polls & 15) return false;
-    if (word_load(flag)) return true;
-    const long long now = (long long)wall_clock64();
-    if (polls == 16) start = now;
-    if (now - start < ticks) return false;
-    word_store(flag, kCgExpired);
+    const int left = word_load(flag);
+    if (!left) {
+      const long long now = (long long)wall_clock64();
+      if (polls == 16) start = now;
+      if (now - start < ticks) return false;
+    }
+    if (decide(verdict, kCgExpired) == kCgDone) return false;
+    if (!left) word_store(flag, kCgExpired);
     return true;
   }
 };
@@ -234,7 +259,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   __shared__ double s_acc[NP][BS / 4 > kAcc ? BS / 4 : kAcc];
   __shared__ double s_tot[NP];
   __shared__ unsigned s_scan[BS / kWave];
-  __shared__ int s_dead;
+  __shared__ int s_dead, s_verdict;
   if (blockIdx.x % A.stride) return;
   const unsigned n = 3u * (unsigned)A.nrows;
   for (int phase = 0; phase < (A.sys ? 2 : 1); ++phase) {
@@ -267,6 +292,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
     sys = CgResidentSys{uniform(q.row0), uniform(q.row1), uniform(q.max_iters), uniform(q.id),
                         q.tol};
   }
+  int* const verdict = A.flag + 1 + sys.id;
   PcgCtrl* const ctrl = A.ctrl + sys.id;
   PcgCtrl* const mirror = A.mirror ? A.mirror + sys.id : nullptr;
   const int nrows = sys.row1 - sys.row0;
@@ -380,7 +406,7 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
   double threshold = 0.0, b2 = 0.0, alpha = 0.0, beta = 0.0;
   int done = kCgExpired;
   for (int it = 0;; ++it) {
-    Waiter wait{A.flag, A.wait_ticks};
+    Waiter wait{A.flag, verdict, A.wait_ticks};
     bool dead = false;
     W w[EPT];
 #pragma unroll
@@ -432,19 +458,29 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
       const int jt = it - 1;  // iteration of the sums
       const bool converged = rr < threshold || b2 == 0.0;
       if (converged || jt >= sys.max_iters) {
-        if (wg == 0 && tid == 0) {
-          PcgCtrl o{};
-          o.rr = rr;
-          o.b2 = b2;
-          o.threshold = threshold;
-          o.iter = converged ? (jt > 0 ? jt - 1 : 0) : jt;
-          o.done = kCgDone;
-          o.max_iters = sys.max_iters;
-          o.stop_it = it;
-          o.started = it;
-          publish_stop(o, ctrl, mirror);
+        if (tid == 0) {
+          int v;
+          if (wg == 0) {
+            v = decide(verdict, kCgDone);
+            if (v == kCgDone) {
+              PcgCtrl o{};
+              o.rr = rr;
+              o.b2 = b2;
+              o.threshold = threshold;
+              o.iter = converged ? (jt > 0 ? jt - 1 : 0) : jt;
+              o.done = kCgDone;
+              o.max_iters = sys.max_iters;
+              o.stop_it = it;
+              o.started = it;
+              publish_stop(o, ctrl, mirror);
+            }
+          } else {
+            while (!(v = word_load(verdict))) __builtin_amdgcn_s_sleep(1);
+          }
+          s_verdict = v;
         }
-        done = kCgDone;
+        __syncthreads();
+        done = s_verdict;
         break;
       }
       // (the two divisions side by side)
@@ -574,7 +610,6 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
     return;
   }
   // the solution (the iterate of the last completed update)
-  __syncthreads();
   for (unsigned o = tid; o < nown; o += BS) A.x[3 * (unsigned)c0 + o] = xl[o];
   }
   }
@@ -583,12 +618,13 @@ __global__ __launch_bounds__(BS) void k_cg_resident(CgResidentArgs<T> A) {
 // Empties the exchange buffers and the flag ahead of a solve.
 template <typename W>
 __global__ __launch_bounds__(256) void k_cg_resident_clear(W* q, long nq, W empty, U64* parts,
-                                                           long np, int* flag, double* x, long nx) {
+                                                           long np, int* flag, int nflag,
+                                                           double* x, long nx) {
   const long i0 = blockIdx.x * 256L + threadIdx.x, step = gridDim.x * 256L;
   for (long i = i0; i < nq; i += step) q[i] = empty;
   for (long i = i0; i < nx; i += step) x[i] = 0.0;  // systems that are not solved
   for (long i = i0; i < np; i += step) parts[i] = kEmpty64;
-  if (i0 == 0) *flag = 0;
+  for (long i = i0; i < nflag; i += step) flag[i] = 0;
 }
 
 constexpr int kBS = 512;  // threads of a workgroup
@@ -664,7 +700,7 @@ void clear(const CgResidentArgs<T>& A, hipStream_t st) {
   const long nq = 9L * A.nrows, np = (A.sys ? 2L : 1L) * 3 * 8 * kCgResidentMaxWg;
   const int gc = (int)std::min<long>(1024, (std::max(nq, np) + 255) / 256);
   hipLaunchKernelGGL(k_cg_resident_clear<W>, dim3(gc), dim3(256), 0, st, A.q, nq, Word<T>::kEmpty,
-                     A.parts, np, A.flag, A.x, A.sys ? 3L * A.nrows : 0L);
+                     A.parts, np, A.flag, 1 + A.nsys, A.x, A.sys ? 3L * A.nrows : 0L);
 }
 
 // The kernel for R passes of rows of at most max_row blocks on nwg workgroups.

@@ -229,7 +229,8 @@ struct CgResidentArgs {
   T* spill = nullptr;          // CgResidentPlan::spill values
   int stride = 1;              // CgResidentPlan::stride
   int lds = 0;                 // dynamic LDS of a workgroup (set by the launch)
-  int* flag = nullptr;
+  int nsys = 1;                // systems (sys), their ids below nsys
+  int* flag = nullptr;         // 1 + nsys words: a workgroup gave up, the verdicts
   PcgCtrl* ctrl = nullptr;
   PcgCtrl* mirror = nullptr;   // as in PcgBuffers; its done is kCgDone or kCgExpired
   // several systems: their list, in the order of the teams that solve them, and

@@ -73,8 +73,9 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 }  // namespace
 
 // Byte layout of the work arrays of one solve on n = 3 nb scalar rows: the
-// control block, the pattern flag, the two partial-sum buffers, D^-1 and the
-// two CG state buffers ({r, q, p, D^-1} per row).
+// control block, the pattern flags and the resident CG's flag and verdict, the
+// two partial-sum buffers, D^-1 and the two CG state buffers ({r, q, p, D^-1}
+// per row).
 struct PcgWorkLayout {
   size_t ctrl = 0, flag = 0, parts = 0, invdiag = 0, state0 = 0, state1 = 0, total = 0;
   explicit PcgWorkLayout(long n) {
@@ -82,7 +83,7 @@ struct PcgWorkLayout {
     ctrl = o;
     o += align256(sizeof(PcgCtrl));
     flag = o;
-    o += align256(3 * sizeof(int));
+    o += align256(4 * sizeof(int));
     parts = o;
     o += align256(sizeof(double) * 2 * kCgParts * (size_t)kCgMaxBlocks);
     invdiag = o;

@@ -18,7 +18,7 @@ import os
 import numpy as np
 import pytest
 
-from mfem_amd import scenes
+from mfem_amd import meshio, scenes
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden")
@@ -161,6 +161,62 @@ def test_expired_wait_falls_back(native, tmp_path):
         out.append((g.positions(), g.stats()["newton_iters"]))
     assert out[0][1] == out[1][1]
     assert np.abs(out[0][0] - out[1][0]).max() < 1e-8
+
+
+def scene_file(tmp_path, n, **kw):
+    """A beam of n cells as a scene file: what resident_wait_ms can be set in."""
+    scene = json.load(open(os.path.join(GOLDEN, "beam_scene.json")))
+    V, T = scenes.kuhn_beam(*n, 0.1, 0.1, 3)
+    meshio.write_mesh(str(tmp_path / "beam.mesh"), V, T)
+    scene["objects"][0]["path"] = str(tmp_path / "beam.mesh")
+    scene.update(kw)
+    path = tmp_path / "scene.json"
+    path.write_text(json.dumps(scene))
+    return str(path)
+
+
+@pytest.mark.parametrize("cap", [1, 2, 3])
+@pytest.mark.parametrize("n", [(3, 1, 1), (20, 6, 6), (40, 13, 13)])
+def test_a_solve_is_whole_whoever_gives_up(native, tmp_path, n, cap):
+    """Short solves in which a workgroup's wait may run out at any point, the
+    last sums included: every row of the step is the iterate of a whole solve
+    (1, 16 and all workgroups). Few iterations from the same data round alike:
+    1e-12."""
+    path = scene_file(tmp_path, n, resident_wait_ms=0, max_iterative_solver_iters=cap,
+                      iterative_solver_tolerance=1e-30)
+
+    def dx(shape):
+        g = native.Sim(json_path=path)
+        if shape is not None:
+            g.set_cg_shape(shape)
+        g.update_system()
+        g.solve()
+        return g.get("dx"), int(g.get_int("pcg_iters")[0])
+
+    want, iters = dx(0)
+    assert np.abs(want).max() > 0 and iters == cap
+    for _ in range(6):
+        got, it = dx(None)
+        assert it == cap
+        assert np.abs(got - want).max() < 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("nb", [1, 40, 2000, 6000])
+def test_solves_that_stop_at_once(native, nb):
+    """b = 0, no iterations allowed, and a tolerance that b itself meets: x is 0
+    in every row, whatever it held."""
+    import torch
+    rp = torch.arange(nb + 1, dtype=torch.int32, device="cuda")
+    col = torch.arange(nb, dtype=torch.int32, device="cuda")
+    K = (2.0 * torch.eye(3, dtype=torch.float64, device="cuda")).repeat(nb, 1, 1).reshape(-1)
+    b = torch.ones(3 * nb, dtype=torch.float64, device="cuda")
+    for rhs, tol, cap in ((0 * b, 1e-6, 10), (b, 1e-6, 0), (b, 2.0, 10)):
+        x = torch.full_like(b, float("nan"))
+        x, it, rr = native.pcg_bsr3(rp, col, K, rhs, tol, cap, x=x)
+        assert it == 0 and rr == (1.0 if rhs is b else 0.0)
+        assert not torch.any(x != 0)
+    x, it, rr = native.pcg_bsr3(rp, col, K, b, 1e-12, 10)
+    assert torch.equal(x, 0.5 * b)
 
 
 @pytest.mark.parametrize("n", [(1, 1, 1), (4, 3, 2), (9, 7, 5), (20, 16, 13), (40, 40, 32)])
