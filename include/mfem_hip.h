@@ -125,7 +125,10 @@ long mfem_sim_size(mfem_sim* sim, const char* name);
 int mfem_sim_get(mfem_sim* sim, const char* name, double* out);
 /* "rowptr", "colind" (scalar CSR pattern), "free_map", "fixed",
  * "bsr_rowptr", "bsr_col", "slot_ptr", "slots", "pcg_iters" (CG iterations
- * of the last solve); "eigen-pcg-IC": "ic_color" (colour of every free
+ * of the last solve); "eigen-pcg-diag": "cg_paths" (CG solves since creation,
+ * a defect-correction sweep being one: by the resident kernel; resident launches
+ * refused, without room for their columns, and expired; by one launch per
+ * iteration); "eigen-pcg-IC": "ic_color" (colour of every free
  * vertex), "ic_colors", "ic_attempts" (factorizations of the last solve) */
 int mfem_sim_get_int(mfem_sim* sim, const char* name, int* out);
 /* The last step's Newton iterations, one row of 10 doubles each: iteration,

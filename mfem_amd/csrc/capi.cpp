@@ -197,6 +197,12 @@ std::vector<int> fetch_int(mfem_sim* sim, const std::string& k) {
   if (k == "slot_ptr") return m.d_slot_ptr.to_host(st);
   if (k == "slots") return m.d_slots.to_host(st);
   if (k == "pcg_iters") return {sim->opt->solver()->stats().iterations};
+  if (k == "cg_paths") {
+    auto* pcg = dynamic_cast<PcgSolver<3>*>(sim->opt->solver());
+    if (!pcg) throw std::runtime_error("no CG solver");
+    const auto& p = pcg->cg_paths();
+    return {p.resident, p.refused, p.no_fit, p.expired, p.launches};
+  }
   if (k == "ic_color" || k == "ic_colors" || k == "ic_attempts") {
     auto* ic = dynamic_cast<IcPcgSolver<3>*>(sim->opt->solver());
     if (!ic) throw std::runtime_error("the linear solver is not \"eigen-pcg-IC\"");
@@ -409,7 +415,7 @@ long mfem_sim_size(mfem_sim* sim, const char* name) {
   int rc = guarded([&] {
     const std::string k(name);
     if (k == "rowptr" || k == "colind" || k == "free_map" || k == "fixed" || k == "bsr_rowptr" ||
-        k == "bsr_col" || k == "slot_ptr" || k == "slots" || k == "pcg_iters" ||
+        k == "bsr_col" || k == "slot_ptr" || k == "slots" || k == "pcg_iters" || k == "cg_paths" ||
         k == "ic_color" || k == "ic_colors" || k == "ic_attempts")
       n = (long)fetch_int(sim, k).size();
     else

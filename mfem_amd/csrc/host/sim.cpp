@@ -616,13 +616,18 @@ bool PcgSolver<DIM>::run_cg_resident(const double* b, double* x, double tol, int
   if (!launch_cg_resident<T>(A, plan.nwg, max_row_, st)) {
     (void)hipGetLastError();
     res_fits_ = false;
+    ++paths_.refused;
     return false;
   }
   // the workgroup that writes the mirror ends whatever the others do
   while (!mirror->done) _mm_pause();
   std::atomic_thread_fence(std::memory_order_acquire);
   if (mirror->done == kCgNoFit) res_fits_ = false;
-  if (mirror->done != kCgDone) return false;
+  if (mirror->done != kCgDone) {
+    ++(mirror->done == kCgNoFit ? paths_.no_fit : paths_.expired);
+    return false;
+  }
+  ++paths_.resident;
   last_ = PcgCtrl{};
   last_.rr = mirror->rr;
   last_.b2 = mirror->b2;
@@ -638,6 +643,7 @@ template <int DIM>
 template <typename T>
 int PcgSolver<DIM>::run_cg(const double* b, double* x, double tol, int max_iters) {
   if (run_cg_resident<T>(b, x, tol, max_iters)) return last_.iter;
+  ++paths_.launches;
   hipStream_t st = this->state_->ctx_->stream;
   PcgBuffers<T> B = buffers<T>(b, x);
   // Every CG kernel that does work writes its index into mapped pinned

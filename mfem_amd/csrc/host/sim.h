@@ -331,6 +331,13 @@ class PcgSolver : public LinearSolver<DIM> {
   int cg_variant() const { return cg_variant_; }
   int cg_blocks() const { return cg_blocks_; }
   const std::vector<CgTrial>& cg_trials() const { return cg_trials_; }
+  // CG solves since creation (a defect-correction sweep is one each): by the
+  // resident kernel; resident launches that were refused, whose columns did not
+  // fit or whose wait expired; by one launch per iteration.
+  struct CgPaths {
+    int resident = 0, refused = 0, no_fit = 0, expired = 0, launches = 0;
+  };
+  const CgPaths& cg_paths() const { return paths_; }
   void force_cg_shape(int variant, int blocks);
   // Profiling stamps of the last two CG launches: [2][blocks][start, end]
   // device wall-clock ticks, and the clock rate in kHz.
@@ -365,6 +372,7 @@ class PcgSolver : public LinearSolver<DIM> {
   bool cg_forced_ = false;  // shape set by force_cg_shape
   int max_row_ = 0;         // blocks in the longest row of K
   bool res_fits_ = true;    // false once the resident CG found that K does not fit
+  CgPaths paths_;
   std::vector<CgTrial> cg_trials_;
   SystemMatrixPD<DIM> system_;
   DeviceArray<double> x_, r64_, dx64_;

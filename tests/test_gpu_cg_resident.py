@@ -42,21 +42,29 @@ def solve(native, sc, precision, shape=None):
     return g.get("dx"), int(g.get_int("pcg_iters")[0]), g
 
 
-def compare(native, sc, precision):
+def paths(g):
+    """How this simulation's CG solves ran (a refused, unfitting or expired
+    resident launch counts as one by launches too)."""
+    return dict(zip(("resident", "refused", "no_fit", "expired", "launches"),
+                    map(int, g.get_int("cg_paths"))))
+
+
+def compare(native, sc, precision, path="resident"):
+    """The default path, which has to be `path`, against the launches."""
     sc.itr_tol = 1e-12 if precision == "fp64" else 1e-10
     sc.max_iters = 20000
     a, ia, g = solve(native, sc, precision)
-    b, ib, _ = solve(native, sc, precision, 0)
+    b, ib, h = solve(native, sc, precision, 0)
+    got, other = paths(g), paths(h)
+    assert got.pop(path) > 0 and other.pop("launches") > 0
+    if path == "no_fit":  # found at the first sweep, which launches took over
+        assert got.pop("launches") > 0
+    assert not any(got.values()) and not any(other.values()), (got, other)
     assert np.isfinite(a).all() and np.abs(b).max() > 0
     assert np.abs(a - b).max() / np.abs(b).max() < 1e-8
     if precision == "fp64":
         assert abs(ia - ib) <= max(3, 0.02 * ib), (ia, ib)
     return g
-
-
-def assert_resident(g):
-    # the other path times its shapes on the first solve from 20,000 rows on
-    assert g.cg_tuning()[0] == []
 
 
 # 1 row per workgroup .. the last size on one XCD, the first over all of them,
@@ -65,18 +73,18 @@ def assert_resident(g):
 @pytest.mark.parametrize("n", [(1, 1, 1), (2, 1, 2), (7, 3, 3), (32, 7, 7), (33, 7, 7), (41, 19, 20),
                                (61, 22, 22), (60, 24, 24), (81, 25, 25), (90, 30, 30)])
 def test_beams(native, n, precision):
-    g = compare(native, scenes.beam_scene(*n, seed=5, mixed=n[0] % 2 == 0), precision)
-    if precision == "mixed" or n[0] < 90:  # 86k rows are past the FP64 kernels
-        assert_resident(g)
+    compare(native, scenes.beam_scene(*n, seed=5, mixed=n[0] % 2 == 0), precision,
+            # 86k rows are past the FP64 kernels
+            "resident" if precision == "mixed" or n[0] < 90 else "launches")
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("n", [(9, 4), (270, 60), (270, 61), (400, 120), (500, 160), (700, 150),
                                (900, 170), (900, 220)])
 def test_sheets(native, n, precision):
-    g = compare(native, scenes.rect2d_scene(*n), precision)
-    if precision == "mixed" or n[0] < 900:
-        assert_resident(g)
+    # 154k and 199k rows are past the FP64 kernels
+    compare(native, scenes.rect2d_scene(*n), precision,
+            "resident" if precision == "mixed" or n[0] < 900 else "launches")
 
 
 def cloud_scene(points, seed, hub=0):
@@ -114,9 +122,64 @@ def cloud_scene(points, seed, hub=0):
 @pytest.mark.parametrize("points,hub", [(6, 0), (16, 0), (27, 0), (0, 50), (0, 90)])
 def test_long_rows(native, points, hub, precision):
     sc = cloud_scene(points, 3, hub)
-    g = compare(native, sc, precision)
-    rows = np.diff(g.get_int("bsr_rowptr"))
+    rows = np.diff(native.Sim(sc).get_int("bsr_rowptr"))
     assert rows.max() > (hub * 0.6 if hub else 16)
+    # 64 or 32 rows a pass on 248 workgroups, 2 (FP64) or 4 passes
+    room = 248 * (64 if rows.max() <= 32 else 32) * (2 if precision == "fp64" else 4)
+    compare(native, sc, precision,
+            "resident" if rows.max() <= 64 and rows.size <= room else "launches")
+
+
+def shuffled(sc, seed):
+    """The same mesh with its vertices in random order: rows of a workgroup then
+    touch columns all over the mesh."""
+    perm = np.random.RandomState(seed).permutation(sc.nV)
+    inv = np.empty_like(perm)
+    inv[perm] = np.arange(sc.nV)
+    sc.V, sc.fixed, sc.T = sc.V[perm], sc.fixed[perm], inv[sc.T].astype(np.int32)
+    return sc
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_columns_that_do_not_fit(native, precision):
+    """37.5k rows, 152 a workgroup, in random order: some 2000 columns a workgroup,
+    and 1365 have room. Every workgroup leaves at the start."""
+    g = compare(native, shuffled(scenes.beam_scene(60, 24, 24, seed=5), 1), precision, "no_fit")
+    g.update_system()
+    g.solve()  # known now: not tried again
+    assert paths(g)["no_fit"] == 1 and paths(g)["resident"] == 0
+
+
+def test_caller_columns_that_do_not_fit(native):
+    """The same through mfem_pcg_bsr3: 40k rows of 13 blocks at random distances.
+    The residual of x itself, to the rounding of K x (about 1e-14)."""
+    import torch
+    rng = np.random.RandomState(2)
+    n, i = 40000, np.arange(40000)
+    A = 0.2 * rng.randn(6, n, 3, 3)
+    W = A @ A.transpose(0, 1, 3, 2) + 0.3 * np.eye(3)
+    far = rng.choice(np.arange(100, n // 2 - 100), 6, replace=False)
+    to = [(i + o) % n for o in far]
+    diag = np.tile(1e-2 * np.eye(3), (n, 1, 1))
+    for w, j in zip(W, to):
+        diag += w
+        diag[j] += w
+    rows = np.concatenate([i] + [i] * 6 + to)
+    cols = np.concatenate([i] + to + [i] * 6)
+    vals = np.concatenate([diag] + [-w for w in W] * 2)
+    order = np.lexsort((cols, rows))
+    rows, cols, vals = rows[order], cols[order], vals[order]
+    rowptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    b = rng.randn(n, 3)
+    dev = [torch.as_tensor(np.ascontiguousarray(a), device="cuda")
+           for a in (rowptr, cols.astype(np.int32), vals.reshape(-1), b.reshape(-1))]
+    x, it, rr = native.pcg_bsr3(*dev, 1e-9, 5000)
+    x = x.cpu().numpy().reshape(-1, 3)
+    r = b.copy()
+    np.subtract.at(r, rows, (vals @ x[cols][:, :, None])[:, :, 0])
+    assert 0 < it < 5000 and rr < 1e-9
+    true = np.linalg.norm(r) / np.linalg.norm(b)
+    assert abs(true - rr) < 1e-14 * np.abs(vals).sum((1, 2)).max() * np.linalg.norm(x) / np.linalg.norm(b) * it
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
@@ -126,7 +189,8 @@ def test_matches_the_oracle(native, oracle, precision):
     o = oracle.Sim(sc)
     o.update_system()
     o.solve()
-    dx, it, _ = solve(native, sc, precision)
+    dx, it, g = solve(native, sc, precision)
+    assert paths(g)["resident"] > 0 and paths(g)["launches"] == 0
     ref = o.get("dx")
     # mixed: K itself is stored in FP32 (2^-24 = 6e-8 an entry), and a solve
     # amplifies that by at most the scaled condition, about 1e2 here
@@ -140,6 +204,7 @@ def test_stopping_rule(native):
         sc = scenes.beam_scene(8, 3, 3, seed=7, mixed=True, **kw)
         a, ia, g = solve(native, sc, "fp64")
         b, ib, _ = solve(native, sc, "fp64", 0)
+        assert paths(g)["resident"] == 1
         assert ia == ib == want
         assert np.allclose(a, b, rtol=0, atol=1e-12 * max(1.0, np.abs(b).max()))
 
@@ -292,3 +357,25 @@ def test_batches(native, sizes, precision):
             # both converge to the same dx (1e-8 of it, see the bars above);
             # positions are of the order of the beam
             assert np.abs(xa - xb).max() < 1e-8 * np.abs(xb).max(), (step, k)
+    # a resident solve is one submission, an iteration of the lockstep CG one each
+    (_, ca, na), (_, cb, _) = a.launch_counts(), b.launch_counts()
+    if precision == "fp64" and (60, 13, 13) in sizes:
+        assert ca > 4 * na
+    else:
+        assert 4 * ca < cb and (ca == na or precision == "mixed")
+
+
+def test_batch_columns_that_do_not_fit(native):
+    """One beam whose columns do not fit its workgroups (9.4k rows, 293 a workgroup,
+    in random order): the whole batch moves to the lockstep CG."""
+    def batch():
+        return native.Batch([scenes.beam_scene(20, 6, 6, seed=1, itr_tol=1e-12, max_iters=20000),
+                             shuffled(scenes.beam_scene(48, 13, 13, seed=2, itr_tol=1e-12,
+                                                        max_iters=20000), 3)], precision="fp64")
+    a, b = batch(), batch()
+    b.set_cg_shape(0, 64)
+    a.step()
+    b.step()
+    for k in range(2):
+        assert np.abs(a.positions(k) - b.positions(k)).max() < 1e-8
+    assert a.launch_counts()[1] > 4 * a.launch_counts()[2]
