@@ -115,7 +115,7 @@ struct SimConfig {
   Precision precision = Precision::FP64;
   double resident_wait_ms = 2000;  // longest wait between the workgroups of the resident
                                    // CG before the solve falls back to one launch per
-                                   // iteration (0: at the first wait)
+                                   // iteration (0: at the first poll that finds nothing)
   int pcg_poll = 16;         // CG iterations launched between host polls (the
                              // Jacobi CG keeps a quarter as many queued ahead)
   double inner_tol = 1e-4;   // relative tolerance of each FP32 inner CG solve (MIXED)

@@ -184,7 +184,7 @@ struct Waiter {
   int polls = 0;
   // true when the wait has to be given up
   __device__ __forceinline__ bool expired() {
-    if (++polls & 15) return false;
+    if ((++polls & 15) && ticks > 0) return false;  // (no time at all: the first poll)
     const int left = word_load(flag);
     if (!left) {
       const long long now = (long long)wall_clock64();

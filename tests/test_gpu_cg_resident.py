@@ -224,6 +224,8 @@ def test_expired_wait_falls_back(native, tmp_path):
         for _ in range(2):
             g.step()
         out.append((g.positions(), g.stats()["newton_iters"]))
+        p = paths(g)
+        assert p["expired"] == p["launches"] and (p["expired"] == 0) == (wait > 0), p
     assert out[0][1] == out[1][1]
     assert np.abs(out[0][0] - out[1][0]).max() < 1e-8
 
@@ -256,6 +258,9 @@ def test_a_solve_is_whole_whoever_gives_up(native, tmp_path, n, cap):
             g.set_cg_shape(shape)
         g.update_system()
         g.solve()
+        p = paths(g)
+        if shape is None and n[0] > 3:  # the first of 16 workgroups always has to wait
+            assert p["expired"] == p["launches"] == 1, p
         return g.get("dx"), int(g.get_int("pcg_iters")[0])
 
     want, iters = dx(0)
