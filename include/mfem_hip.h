@@ -225,9 +225,16 @@ int mfem_batch_get_positions(mfem_batch* batch, int sim, double* out);
 int mfem_batch_stats(mfem_batch* batch, int* newton_iters, int* pcg_iters, int* refinements,
                      int* ls_fail, double* decrement, double* step_ms);
 /* Batched CG shape (as mfem_sim_set_cg_shape) and rows per workgroup;
- * variant -1 restores autotuning on the next solve. */
+ * variant -1 restores the default: the resident kernel where every beam fits
+ * its team, else autotuning on the next solve. */
 int mfem_batch_set_cg_shape(mfem_batch* batch, int variant, int rows_per_workgroup);
+/* The forced or tuned shape and rows per workgroup; variant -1 while there is
+ * none (the resident kernel solves). */
 int mfem_batch_cg_shape(mfem_batch* batch, int* variant, int* rows_per_workgroup);
+/* Longest wait in ms between the workgroups of the resident CG before a solve
+ * falls back to one launch per iteration (a scene file's "resident_wait_ms";
+ * default 2000, 0 at the first poll that finds nothing). */
+int mfem_batch_set_resident_wait(mfem_batch* batch, double ms);
 /* hipGraph replay of the batch's Newton phases (no counterpart in the
  * reference; off by default): with on = 1 the element update + assembly phase of every
  * Newton iteration is one captured graph from the second step on, and CG

@@ -761,6 +761,13 @@ int mfem_batch_set_cg_shape(mfem_batch* b, int variant, int rows_per_workgroup) 
   return guarded([&] { b->sim->force_cg_shape(variant, rows_per_workgroup); });
 }
 
+int mfem_batch_set_resident_wait(mfem_batch* b, double ms) {
+  return guarded([&] {
+    if (!(ms >= 0)) throw std::invalid_argument("the wait must be >= 0 ms");
+    b->sim->set_resident_wait(ms);
+  });
+}
+
 int mfem_batch_set_graphs(mfem_batch* b, int on) {
   return guarded([&] { b->sim->set_graphs(on != 0); });
 }

@@ -220,7 +220,10 @@ void BatchSim::force_cg_shape(int variant, int rows_per_wg) {
   rows_per_wg_ = variant < 0 ? 0 : rows_per_wg;
   cg_forced_ = variant >= 0;
   if (variant >= 0) layout_workgroups(rows_per_wg_);
+  else nwg_ = 0;  // a forced layout goes with its shape
 }
+
+void BatchSim::set_resident_wait(double ms) { state_->config_->resident_wait_ms = ms; }
 
 // Workgroups per simulation: ceil(rows / rows_per_wg), at least one.
 void BatchSim::layout_workgroups(int rows_per_wg) {
@@ -246,6 +249,8 @@ void BatchSim::layout_workgroups(int rows_per_wg) {
 template <typename T>
 BatchCgBuffers<T> BatchSim::buffers(const double* b, double* x) {
   auto& m = *state_->mesh_;
+  if (nwg_ <= 0 || (m.nfree() > 0 && (!state0_.template as<T>() || !state1_.template as<T>())))
+    throw std::logic_error("batch: lockstep CG without its buffers or layout");
   BatchCgBuffers<T> B;
   B.n = 3 * m.nfree();
   B.rowptr = m.d_rowptr.data();
@@ -402,7 +407,7 @@ void BatchSim::run_cg(const double* b, double* x, const std::vector<double>& tol
                       const std::vector<int>& budget, const std::vector<int>& on,
                       std::vector<int>& iters) {
   if (run_cg_resident<T>(b, x, tol, budget, on, iters)) return;
-  if (nwg_ == 0) prepare_lockstep<T>();
+  prepare_lockstep<T>();
   auto& S = *state_;
   hipStream_t st = S.ctx_->stream;
   const BatchCgBuffers<T> B = buffers<T>(b, x);
@@ -589,7 +594,6 @@ void BatchSim::tune() {
   layout_workgroups(rows_per_wg_);
 }
 
-// The workgroup layout of the lockstep CG.
 template <typename T>
 void BatchSim::prepare_lockstep() {
   auto& S = *state_;

@@ -45,6 +45,9 @@ class BatchSim {
   int rows_per_workgroup() const { return rows_per_wg_; }
   // Force the CG shape and rows per workgroup (variant -1: autotune again).
   void force_cg_shape(int variant, int rows_per_wg);
+  // Longest wait between the workgroups of the resident CG in ms
+  // (SimConfig::resident_wait_ms).
+  void set_resident_wait(double ms);
   // Replay the element-update + assembly phase and groups of 16 CG
   // iterations as captured hipGraphs; results are identical either way.
   void set_graphs(bool on);
@@ -82,6 +85,8 @@ class BatchSim {
                        const std::vector<int>& budget, const std::vector<int>& on,
                        std::vector<int>& iters);
   int resident_passes(int value_bytes);
+  // Buffers, kernel shape and workgroup layout of the lockstep CG; does nothing
+  // where they are there.
   template <typename T>
   void prepare_lockstep();
   template <typename T>

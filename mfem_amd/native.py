@@ -31,7 +31,7 @@ EXPORTED = [
     "mfem_batch_create", "mfem_batch_destroy", "mfem_batch_step", "mfem_batch_sizes",
     "mfem_batch_get_positions", "mfem_batch_stats", "mfem_batch_set_cg_shape",
     "mfem_batch_cg_shape", "mfem_sim_set_callback", "mfem_pcg_bsr3", "mfem_pcg_bsr3_noalloc",
-    "mfem_batch_set_graphs", "mfem_batch_launch_counts",
+    "mfem_batch_set_graphs", "mfem_batch_launch_counts", "mfem_batch_set_resident_wait",
 ]
 
 # scalar-row limit of mfem_pcg_bsr3_noalloc (MFEM_PCG_NOALLOC_MAX_ROWS)
@@ -123,6 +123,7 @@ def lib():
         L.mfem_batch_stats.argtypes = [vp, ip, ip, ip, ip, dp, dp]
         L.mfem_batch_set_cg_shape.argtypes = [vp, C.c_int, C.c_int]
         L.mfem_batch_cg_shape.argtypes = [vp, ip, ip]
+        L.mfem_batch_set_resident_wait.argtypes = [vp, C.c_double]
         L.mfem_batch_set_graphs.argtypes = [vp, C.c_int]
         L.mfem_batch_launch_counts.argtypes = [vp, C.POINTER(C.c_long), C.POINTER(C.c_long),
                                                C.POINTER(C.c_long)]
@@ -418,6 +419,9 @@ class Batch:
         v, r = C.c_int(), C.c_int()
         check(lib().mfem_batch_cg_shape(self.h, C.byref(v), C.byref(r)))
         return v.value, r.value
+
+    def set_resident_wait(self, ms):
+        check(lib().mfem_batch_set_resident_wait(self.h, float(ms)))
 
     def set_graphs(self, on):
         check(lib().mfem_batch_set_graphs(self.h, int(bool(on))))

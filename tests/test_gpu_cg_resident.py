@@ -370,6 +370,38 @@ def test_batches(native, sizes, precision):
         assert 4 * ca < cb and (ca == na or precision == "mixed")
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("sequence", ["fresh", "restored", "used"])
+def test_batch_falls_back_in_any_state(native, precision, sequence):
+    """A resident launch that gives up while the lockstep CG is not set up: nothing
+    done before, a shape forced and released, and solves of the other kind in
+    between. Its buffers are made then, and the step is the forced batch's."""
+    kw = dict(itr_tol=1e-12 if precision == "fp64" else 1e-10, max_iters=20000, max_newton=3,
+              mixed=True)
+    scs = [scenes.beam_scene(*n, seed=k, **kw)
+           for k, n in enumerate([(20, 6, 6), (5, 2, 3), (33, 9, 8)])]
+    a, b = native.Batch(scs, precision=precision), native.Batch(scs, precision=precision)
+    b.set_cg_shape(0, 256)
+    if sequence != "fresh":
+        a.set_cg_shape(0, 64)
+        if sequence == "used":
+            a.step()
+            b.step()
+        a.set_cg_shape(-1)
+    for wait in (0, 2000, 0):
+        a.set_resident_wait(wait)
+        before = a.launch_counts()
+        a.step()
+        b.step()
+        cg, newton = (x - y for x, y in zip(a.launch_counts()[1:], before[1:]))
+        assert (cg > 20 * newton) == (wait == 0), (wait, cg, newton)
+        for k in range(a.count):
+            xa, xb = a.positions(k), b.positions(k)
+            assert np.abs(xa - xb).max() < 1e-8 * np.abs(xb).max(), k
+    with pytest.raises(native.MfemError, match="wait"):
+        a.set_resident_wait(-1.0)
+
+
 def test_batch_columns_that_do_not_fit(native):
     """One beam whose columns do not fit its workgroups (9.4k rows, 293 a workgroup,
     in random order): the whole batch moves to the lockstep CG."""
