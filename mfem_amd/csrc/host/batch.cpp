@@ -20,6 +20,7 @@ enum { RES_DX = 0, RES_DS = 1, RES_E0 = 2, RES_E1 = 3, RES_ROWS = 4 };
 // pinned staging regions of the small uploads
 enum { ST_TOL, ST_BUDGET, ST_ON_CG, ST_ALPHA0, ST_ON0, ST_ALPHA1, ST_ON1, ST_ACCEPT, kStageRegions };
 constexpr int kTuneMinRows = 20000;
+constexpr int kDefaultRows = 256;  // rows per workgroup where none were tuned
 // CG iteration pairs per replayed graph (16 iterations: one host poll's worth)
 constexpr int kCgGraphPairs = 8;
 }  // namespace
@@ -407,7 +408,7 @@ void BatchSim::run_cg(const double* b, double* x, const std::vector<double>& tol
                       const std::vector<int>& budget, const std::vector<int>& on,
                       std::vector<int>& iters) {
   if (run_cg_resident<T>(b, x, tol, budget, on, iters)) return;
-  prepare_lockstep<T>();
+  prepare_lockstep<T>(false);
   auto& S = *state_;
   hipStream_t st = S.ctx_->stream;
   const BatchCgBuffers<T> B = buffers<T>(b, x);
@@ -544,7 +545,7 @@ void BatchSim::tune() {
   hipStream_t st = S.ctx_->stream;
   if (S.mesh_->nfree() < kTuneMinRows) {
     variant_ = 0;
-    rows_per_wg_ = 256;
+    rows_per_wg_ = kDefaultRows;
     layout_workgroups(rows_per_wg_);
     return;
   }
@@ -554,7 +555,7 @@ void BatchSim::tune() {
   const std::vector<double> tol(nsim_, 0.0);
   const std::vector<int> budget(nsim_, 1 << 30), on(nsim_, 1);
   double best = 1e300;
-  int best_v = 0, best_r = 256;
+  int best_v = 0, best_r = kDefaultRows;
   for (int v = 0; v < cg_variant_count(); ++v) {
     int G, U, BS;
     cg_variant_shape(v, &G, &U, &BS);
@@ -595,13 +596,13 @@ void BatchSim::tune() {
 }
 
 template <typename T>
-void BatchSim::prepare_lockstep() {
+void BatchSim::prepare_lockstep(bool tuned) {
   auto& S = *state_;
   const size_t n = 3 * (size_t)S.mesh_->nfree();
   state0_.resize(4 * n, sizeof(T) == 4);
   state1_.resize(4 * n, sizeof(T) == 4);
-  if (variant_ < 0) tune<T>();
-  else if (nwg_ == 0) layout_workgroups(rows_per_wg_);
+  if (variant_ < 0 && tuned) tune<T>();
+  else if (nwg_ == 0) layout_workgroups(kDefaultRows);
 }
 
 // Linear solve of every simulation that is on (PcgSolver::solve per system:
@@ -616,8 +617,8 @@ void BatchSim::solve(const std::vector<int>& on) {
   const bool f32 = S.ctx_->fp32();
   x_.resize(n);
   if (resident_passes(f32 ? 4 : 8) == 0) {
-    if (f32) prepare_lockstep<float>();
-    else prepare_lockstep<double>();
+    if (f32) prepare_lockstep<float>(true);
+    else prepare_lockstep<double>(true);
   }
   solve_iters_.assign(nsim_, 0);
   solve_sweeps_.assign(nsim_, 0);

@@ -85,10 +85,11 @@ class BatchSim {
                        const std::vector<int>& budget, const std::vector<int>& on,
                        std::vector<int>& iters);
   int resident_passes(int value_bytes);
-  // Buffers, kernel shape and workgroup layout of the lockstep CG; does nothing
-  // where they are there.
+  // Buffers and workgroup layout of the lockstep CG, and with `tuned` its kernel
+  // shape by trials, which overwrite x_: only ahead of a solve. Does nothing where
+  // they are there.
   template <typename T>
-  void prepare_lockstep();
+  void prepare_lockstep(bool tuned);
   template <typename T>
   void tune();
   void layout_workgroups(int rows_per_wg);

@@ -402,6 +402,22 @@ def test_batch_falls_back_in_any_state(native, precision, sequence):
         a.set_resident_wait(-1.0)
 
 
+def test_batch_tunes_ahead_of_a_solve_only(native):
+    """21k rows, enough for the tuner, whose trials overwrite the solution: the
+    solve that falls back has one in progress (the sum of its sweeps) and takes the
+    default shape; the tuner runs ahead of a solve by launches."""
+    scs = [scenes.beam_scene(50, 14, 13 + k, seed=k, itr_tol=1e-10, max_iters=20000, max_newton=1,
+                             mixed=True) for k in range(2)]
+    a, b = native.Batch(scs, precision="mixed"), native.Batch(scs, precision="mixed")
+    b.set_cg_shape(0, 256)
+    a.set_resident_wait(0)
+    a.step()
+    b.step()
+    assert a.launch_counts()[1] > 20 and a.cg_shape() == (-1, 0)
+    for k in range(2):
+        assert np.abs(a.positions(k) - b.positions(k)).max() < 1e-8 * np.abs(b.positions(k)).max()
+
+
 def test_batch_columns_that_do_not_fit(native):
     """One beam whose columns do not fit its workgroups (9.4k rows, 293 a workgroup,
     in random order): the whole batch moves to the lockstep CG."""
