@@ -224,7 +224,10 @@ void BatchSim::force_cg_shape(int variant, int rows_per_wg) {
   else nwg_ = 0;  // a forced layout goes with its shape
 }
 
-void BatchSim::set_resident_wait(double ms) { state_->config_->resident_wait_ms = ms; }
+void BatchSim::set_resident_wait(double ms) {
+  state_->config_->resident_wait_ms = ms;
+  res_backoff_ = ResidentBackoff();
+}
 
 // Workgroups per simulation: ceil(rows / rows_per_wg), at least one.
 void BatchSim::layout_workgroups(int rows_per_wg) {
@@ -276,7 +279,7 @@ BatchCgBuffers<T> BatchSim::buffers(const double* b, double* x) {
 }
 
 int BatchSim::resident_passes(int value_bytes) {
-  if (cg_forced_ || !res_fits_) return 0;
+  if (cg_forced_ || !res_fits_ || !res_backoff_.open()) return 0;
   if (res_passes_ < 0) {
     const auto& rp = state_->mesh_->rowptr_;
     for (size_t i = 0; i + 1 < rp.size(); ++i) max_row_ = std::max(max_row_, rp[i + 1] - rp[i]);
@@ -380,7 +383,10 @@ bool BatchSim::run_cg_resident(const double* b, double* x, const std::vector<dou
     if (mirror[k].done == kCgNoFit) res_fits_ = false;
   }
   if (!launched) res_fits_ = false;
-  if (!ok) return false;
+  if (!ok) {
+    if (res_fits_) res_backoff_.expired();
+    return false;
+  }
   ++subs_cg_;
   iters.assign(nsim_, 0);
   for (int k = 0; k < nsim_; ++k) {
@@ -616,6 +622,7 @@ void BatchSim::solve(const std::vector<int>& on) {
   const int n = 3 * m.nfree();
   const bool f32 = S.ctx_->fp32();
   x_.resize(n);
+  res_backoff_.begin_solve();
   if (resident_passes(f32 ? 4 : 8) == 0) {
     if (f32) prepare_lockstep<float>(true);
     else prepare_lockstep<double>(true);

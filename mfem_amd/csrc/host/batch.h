@@ -120,6 +120,7 @@ class BatchSim {
   std::vector<mfemhip::PcgCtrl> ctrl_host_;
   // resident CG: see CgResidentArgs
   bool cg_forced_ = false, res_fits_ = true;
+  ResidentBackoff res_backoff_;
   int res_passes_ = -1, max_row_ = 0;
   long res_spill_n_ = 0;
   RealArray res_q_, res_spill_;

@@ -578,7 +578,8 @@ PcgBuffers<T> PcgSolver<DIM>::buffers(const double* b, double* x) {
 // one-kernel-per-iteration CG.
 template <int DIM>
 CgResidentPlan PcgSolver<DIM>::resident_plan(int value_bytes) const {
-  if (cg_forced_ || this->profile_spmv || !res_fits_) return CgResidentPlan();
+  if (cg_forced_ || this->profile_spmv || !res_fits_ || !res_backoff_.open())
+    return CgResidentPlan();
   return cg_resident_plan(this->state_->mesh_->nfree(), max_row_, value_bytes);
 }
 
@@ -622,9 +623,14 @@ bool PcgSolver<DIM>::run_cg_resident(const double* b, double* x, double tol, int
   // the workgroup that writes the mirror ends whatever the others do
   while (!mirror->done) _mm_pause();
   std::atomic_thread_fence(std::memory_order_acquire);
-  if (mirror->done == kCgNoFit) res_fits_ = false;
+  if (mirror->done == kCgNoFit) {
+    res_fits_ = false;
+    ++paths_.no_fit;
+    return false;
+  }
   if (mirror->done != kCgDone) {
-    ++(mirror->done == kCgNoFit ? paths_.no_fit : paths_.expired);
+    res_backoff_.expired();
+    ++paths_.expired;
     return false;
   }
   ++paths_.resident;
@@ -808,6 +814,7 @@ void PcgSolver<DIM>::solve() {
   state1_.resize(4 * (size_t)n, f32);
   this->stats_ = SolveStats();
   rf_ = Refinement();
+  res_backoff_.begin_solve();
   if (variant_ < 0) {
     if (f32) tune_spmv<float>();
     else tune_spmv<double>();

@@ -10,6 +10,7 @@
 // control flow (Newton loop, line search, termination tests), exactly as the
 // reference's NewtonOptimizer does.
 #pragma once
+#include <algorithm>
 #include <array>
 #include <functional>
 #include <memory>
@@ -305,6 +306,23 @@ class LinearSolver {
   bool defer_ = false;
 };
 
+// Solves that keep to launches after a wait of the resident CG expired. What makes
+// one expire (another process on the GPU holding part of its CUs) tends to last,
+// and each try costs the whole wait: the next 64 solves don't try, and twice as many
+// after each further expiry.
+class ResidentBackoff {
+ public:
+  void begin_solve() { skip_ -= skip_ > 0; }
+  bool open() const { return skip_ == 0; }
+  void expired() {
+    skip_ = next_ + 1;
+    next_ = std::min(2 * next_, 1 << 20);
+  }
+
+ private:
+  int skip_ = 0, next_ = 64;
+};
+
 // "eigen-pcg-diag": Jacobi-preconditioned CG with Eigen's stopping rule.
 // FP64: one CG solve on the FP64 system. MIXED: FP32 CG sweeps inside an FP64
 // defect-correction loop that stops on the true FP64 residual.
@@ -372,6 +390,7 @@ class PcgSolver : public LinearSolver<DIM> {
   bool cg_forced_ = false;  // shape set by force_cg_shape
   int max_row_ = 0;         // blocks in the longest row of K
   bool res_fits_ = true;    // false once the resident CG found that K does not fit
+  ResidentBackoff res_backoff_;
   CgPaths paths_;
   std::vector<CgTrial> cg_trials_;
   SystemMatrixPD<DIM> system_;

@@ -156,7 +156,9 @@ void pcg_bsr3_run(char* work, int nb, int nnzb, const int* rowptr, const int* co
     MFEM_HIP_CHECK(hipGetDevice(&dev));
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)
       khz = 100000;
-    A.wait_ticks = 2000LL * khz;
+    // no call knows whether the one before waited in vain (see ResidentBackoff), so
+    // the wait is short; on a GPU of its own a workgroup waits for microseconds
+    A.wait_ticks = 100LL * khz;
     if (launch_cg_resident(A, plan.nwg, hflag[1], st)) {
       MFEM_HIP_CHECK(hipMemcpyAsync(&h, A.ctrl, sizeof(PcgCtrl), hipMemcpyDeviceToHost, st));
       MFEM_HIP_CHECK(hipStreamSynchronize(st));
