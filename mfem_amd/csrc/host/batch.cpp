@@ -459,20 +459,25 @@ void BatchSim::run_cg(const double* b, double* x, const std::vector<double>& tol
   // every kernel that read the slot's previous list has then completed, and
   // so has the copy of that list from its pinned source
   long free_from[3] = {0, 0, 0};
+  std::vector<int> live;
   auto compact = [&](long started) {
     if (graphs_) return;
     const int cur = Bc.active ? Bc.nactive : nwg_;
+    // one look at each flag: a system may stop between two of them
+    live.clear();
     int count = 0;
     for (int k = 0; k < nsim_; ++k)
-      if (!mirror[k].done) count += wg0_[k + 1] - wg0_[k];
+      if (!mirror[k].done) {
+        live.push_back(k);
+        count += wg0_[k + 1] - wg0_[k];
+      }
     if (count == 0 || count > cur * 3 / 4) return;
     const int slot = (list_slot + 1) % 3;
     if (started < free_from[slot]) return;
     int* h = pinned_active_->as<int>() + (size_t)slot * nwg_;
     int n = 0;
-    for (int k = 0; k < nsim_; ++k)
-      if (!mirror[k].done)
-        for (int w = wg0_[k]; w < wg0_[k + 1]; ++w) h[n++] = w;
+    for (int k : live)
+      for (int w = wg0_[k]; w < wg0_[k + 1]; ++w) h[n++] = w;
     MFEM_HIP_CHECK(hipMemcpyAsync(d_active_[slot].data(), h, sizeof(int) * (size_t)n,
                                   hipMemcpyHostToDevice, st));
     if (list_slot >= 0) free_from[list_slot] = launched;

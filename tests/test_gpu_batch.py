@@ -123,3 +123,17 @@ def test_batch_graph_replay_is_bit_identical_at_256_beams(native):
     # the first step runs eagerly (its buffers are allocated), then one graph
     assert ug < ue and ug >= ng
     assert cg < 0.2 * ce
+
+
+def test_systems_that_stop_together(native):
+    """40 copies each of 32 beams, mixed precision: many stop in the same few
+    launches, between two looks that the host takes at their flags while it lists
+    the workgroups still running. Copies stay equal."""
+    base = [scenes.beam_scene(12, 3, 3, seed=k, E=10.0 ** (4 + k % 4), mixed=True)
+            for k in range(32)]
+    b = native.Batch(base * 40, precision="mixed")
+    b.set_cg_shape(0, 64)
+    for step in range(20):
+        b.step()
+    for k in range(32):
+        assert np.array_equal(b.positions(k), b.positions(k + 32 * 39))
