@@ -289,6 +289,41 @@ int BatchSim::resident_passes(int value_bytes) {
   return res_passes_;
 }
 
+double BatchSim::resident_us(int rows, double iters) const {
+  return (iters + 4.0) * (3.0 + rows / (64.0 * cg_team_of(rows, nsim_)));
+}
+
+// Whether the resident CG solves these systems sooner than lockstep launches, for
+// the iterations of the last solve (before there is one: resident). Teams work
+// through the systems one after another, 8 or 32 at a time; a lockstep launch costs
+// about 10 us and then streams the blocks and vectors of every running system at
+// about 4.8 TB/s. Many small systems are few iterations in lockstep and many solves
+// one after another for a team. ms of a step, resident against lockstep, FP64 (FP32
+// in brackets): 128 systems of 96 rows 6.3 / 8.5 (5.9 / 7.9), 512 of them 21.8 / 11.8
+// (21.2 / 9.8), 2048 of them 80.8 / 28.1 (77.9 / 22.7); 512 of 980 rows 73 / 141 (66 /
+// 86); 128 of 1280 rows, each on a whole XCD, 51.6 / 56.6 (48.2 / 40.4), 400 of them
+// 160 / 145 (151 / 88); 64 of 9900 rows 104 / 223 (69 / 129). The estimates agree with
+// these within a fifth.
+bool BatchSim::resident_pays(const std::vector<int>& on, int value_bytes) const {
+  if (last_iters_.empty()) return true;
+  constexpr double kLaunchUs = 9.7, kBytesPerUs = 4.8e6;
+  const auto& rp = state_->mesh_->rowptr_;
+  double large = 0, small = 0, longest = 0, bytes = 0, launches = 0;
+  for (int k = 0; k < nsim_; ++k) {
+    const int rows = f0_[k + 1] - f0_[k];
+    if (!on[k] || rows == 0) continue;
+    const double us = resident_us(rows, last_iters_[k]);
+    (cg_team_of(rows, nsim_) == kCgTeamLarge ? large : small) += us;
+    longest = std::max(longest, us);
+    launches = std::max(launches, (double)last_iters_[k]);
+    bytes += last_iters_[k] * ((rp[f0_[k + 1]] - rp[f0_[k]]) * (9.0 * value_bytes + 4.0) +
+                              rows * (24.0 * value_bytes + 48.0));
+  }
+  const double resident =
+      std::max(longest, (large * kCgTeamLarge + small * kCgTeamSmall) / kCgResidentMaxWg);
+  return resident <= launches * kLaunchUs + bytes / kBytesPerUs;
+}
+
 template <typename T>
 bool BatchSim::run_cg_resident(const double* b, double* x, const std::vector<double>& tol,
                                const std::vector<int>& budget, const std::vector<int>& on,
@@ -307,8 +342,7 @@ bool BatchSim::run_cg_resident(const double* b, double* x, const std::vector<dou
   auto cost = [&](int k) {
     const int rows = f0_[k + 1] - f0_[k];
     const double it = res_cost_[k] > 0 ? res_cost_[k] : 50.0 + std::cbrt((double)rows) * 5.0;
-    return (std::min<double>(it, budget[k]) + 4.0) *
-           (3.0 + rows / (64.0 * cg_team_of(rows, nsim_)));
+    return resident_us(rows, std::min<double>(it, budget[k]));
   };
   std::vector<int> order;
   for (int k = 0; k < nsim_; ++k)
@@ -413,7 +447,7 @@ template <typename T>
 void BatchSim::run_cg(const double* b, double* x, const std::vector<double>& tol,
                       const std::vector<int>& budget, const std::vector<int>& on,
                       std::vector<int>& iters) {
-  if (run_cg_resident<T>(b, x, tol, budget, on, iters)) return;
+  if (use_resident_ && run_cg_resident<T>(b, x, tol, budget, on, iters)) return;
   prepare_lockstep<T>(false);
   auto& S = *state_;
   hipStream_t st = S.ctx_->stream;
@@ -628,7 +662,8 @@ void BatchSim::solve(const std::vector<int>& on) {
   const bool f32 = S.ctx_->fp32();
   x_.resize(n);
   res_backoff_.begin_solve();
-  if (resident_passes(f32 ? 4 : 8) == 0) {
+  use_resident_ = resident_passes(f32 ? 4 : 8) > 0 && resident_pays(on, f32 ? 4 : 8);
+  if (!use_resident_) {
     if (f32) prepare_lockstep<float>(true);
     else prepare_lockstep<double>(true);
   }
@@ -692,6 +727,9 @@ void BatchSim::solve(const std::vector<int>& on) {
       launch_axpy(n, 1.0, dx64_.data(), x_.data(), st);
     }
   }
+  last_iters_.resize(nsim_, 1);
+  for (int k = 0; k < nsim_; ++k)
+    if (on[k]) last_iters_[k] = std::max(1, solve_iters_[k]);
   system_.post_solve(&S, x_.data());
 }
 

@@ -85,6 +85,9 @@ class BatchSim {
                        const std::vector<int>& budget, const std::vector<int>& on,
                        std::vector<int>& iters);
   int resident_passes(int value_bytes);
+  // us that the resident CG takes on a system of `rows` rows and `iters` iterations
+  double resident_us(int rows, double iters) const;
+  bool resident_pays(const std::vector<int>& on, int value_bytes) const;
   // Buffers and workgroup layout of the lockstep CG, and with `tuned` its kernel
   // shape by trials, which overwrite x_: only ahead of a solve. Does nothing where
   // they are there.
@@ -120,6 +123,7 @@ class BatchSim {
   std::vector<mfemhip::PcgCtrl> ctrl_host_;
   // resident CG: see CgResidentArgs
   bool cg_forced_ = false, res_fits_ = true;
+  bool use_resident_ = false;  // in this solve
   ResidentBackoff res_backoff_;
   int res_passes_ = -1, max_row_ = 0;
   long res_spill_n_ = 0;
@@ -129,7 +133,8 @@ class BatchSim {
   DeviceArray<mfemhip::CgResidentSys> res_sys_;
   std::unique_ptr<PinnedBuffer> res_stage_;  // source of res_sys_ and res_team_
   double wall_khz_ = 100000.0;               // device wall-clock rate
-  std::vector<double> res_cost_;             // iterations of each system's last solve
+  std::vector<double> res_cost_;             // iterations of each system's last sweep
+  std::vector<int> last_iters_;              // and of its last solve (resident_pays)
   // mapped copy of every system's control block, then the progress word
   std::unique_ptr<PinnedBuffer> pinned_ctrl_;
   // Compacted lists of the workgroups of the systems still iterating (eager

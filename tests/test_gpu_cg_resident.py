@@ -383,6 +383,29 @@ def test_batches(native, sizes, precision):
         assert 4 * ca < cb and (ca == na or precision == "mixed")
 
 
+@pytest.mark.parametrize("precision,n,count,resident", [
+    ("fp64", (6, 3, 3), 32, True), ("fp64", (6, 3, 3), 1024, False),
+    ("mixed", (6, 3, 3), 1024, False), ("mixed", (20, 7, 7), 16, True),
+    ("mixed", (20, 7, 7), 320, False), ("fp64", (20, 6, 6), 128, True)])
+def test_batch_takes_the_shorter_way(native, precision, n, count, resident):
+    """Many small beams are few iterations in lockstep and many solves one after
+    another for a team: from the second solve on, when the iterations are known, the
+    batch goes the way that is shorter by a factor of two or so either way."""
+    kw = dict(itr_tol=1e-8, max_iters=2000, max_newton=2, mixed=True)
+    base = [scenes.beam_scene(*n, seed=k, E=10.0 ** (4 + k % 4), **kw) for k in range(8)]
+    a, b = (native.Batch(base * (count // 8), precision=precision) for _ in range(2))
+    b.set_cg_shape(0, 64)
+    a.step()
+    b.step()
+    before = a.launch_counts()
+    a.step()
+    b.step()
+    cg, newton = (x - y for x, y in zip(a.launch_counts()[1:], before[1:]))
+    assert (cg <= 8 * newton) if resident else (cg > 20 * newton), (cg, newton)
+    for k in (0, 7, count - 1):
+        assert np.abs(a.positions(k) - b.positions(k)).max() < 1e-6 * np.abs(b.positions(k)).max()
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("sequence", ["fresh", "restored", "used"])
 def test_batch_falls_back_in_any_state(native, precision, sequence):
