@@ -399,6 +399,7 @@ bool BatchSim::run_cg_resident(const double* b, double* x, const std::vector<dou
   A.parts = res_parts_.data();
   A.spill = res_spill_.template as<T>();
   A.nsys = nsim_;
+  for (int k = 0; k < nsim_; ++k) A.sys_rows = std::max(A.sys_rows, f0_[k + 1] - f0_[k]);
   A.flag = res_flag_.data();
   A.ctrl = ctrls_.data();
   A.mirror = pinned_ctrl_->device<PcgCtrl>();

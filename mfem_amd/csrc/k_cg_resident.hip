@@ -636,7 +636,9 @@ bool launch_shape(const CgResidentArgs<T>& A, int nwg, hipStream_t st) {
   using L = ResidentLds<R, NLDS, EPT, BS, G, T>;
   static_assert(L::p < kLdsBytes, "LDS");
   if (NREG + NLDS < R * U && !A.spill) return false;
-  if (L::start + 8L * ((A.nrows + 31) / 32) > kLdsBytes) return false;
+  // the bit set that numbers one system's columns, and its ranks
+  const long rows = A.sys ? A.sys_rows : A.nrows;
+  if (L::start + 8L * ((rows + 31) / 32) > kLdsBytes) return false;
   const void* f = reinterpret_cast<const void*>(
       &k_cg_resident<G, U, R, NREG, NLDS, EPT, BS, T>);
   if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess)

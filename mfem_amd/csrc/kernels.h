@@ -230,6 +230,7 @@ struct CgResidentArgs {
   int stride = 1;              // CgResidentPlan::stride
   int lds = 0;                 // dynamic LDS of a workgroup (set by the launch)
   int nsys = 1;                // systems (sys), their ids below nsys
+  int sys_rows = 0;            // block rows of the largest system (nrows without sys)
   int* flag = nullptr;         // 1 + nsys words: a workgroup gave up, the verdicts
   PcgCtrl* ctrl = nullptr;
   PcgCtrl* mirror = nullptr;   // as in PcgBuffers; its done is kCgDone or kCgExpired

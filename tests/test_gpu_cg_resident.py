@@ -406,6 +406,20 @@ def test_batch_takes_the_shorter_way(native, precision, n, count, resident):
         assert np.abs(a.positions(k) - b.positions(k)).max() < 1e-6 * np.abs(b.positions(k)).max()
 
 
+def test_batch_of_many_beams_is_resident(native):
+    """A beam's place on its team depends on its own rows, not on the batch's: 640
+    beams of 980 rows, 627k in all. The first and last against the lockstep CG."""
+    scs = [scenes.beam_scene(20, 6, 6, seed=k, E=10.0 ** (4 + k % 4), itr_tol=1e-12,
+                             max_iters=20000, max_newton=1, mixed=True) for k in range(8)] * 80
+    a, b = native.Batch(scs, precision="fp64"), native.Batch(scs, precision="fp64")
+    b.set_cg_shape(0, 256)
+    a.step()
+    b.step()
+    assert a.launch_counts()[1] == a.launch_counts()[2] == 1
+    for k in (0, 7, 632, 639):
+        assert np.abs(a.positions(k) - b.positions(k)).max() < 1e-8 * np.abs(b.positions(k)).max()
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("sequence", ["fresh", "restored", "used"])
 def test_batch_falls_back_in_any_state(native, precision, sequence):
