@@ -1313,16 +1313,28 @@ __global__ __launch_bounds__(kElemBlock) void k_plain2d_energy(
 // ---------------------------------------------------------------------------
 // Batched element evaluations (points in AoS, column-major per point).
 // Records of the batched entry points (element-major, N values each) pass
-// through LDS, so that a wave reads and writes contiguous runs: from every lane
-// a record of its own would touch 64 cache lines per instruction. An odd pitch
-// keeps the LDS banks apart. One wave per workgroup.
+// through LDS where there are many, so that a wave reads and writes contiguous
+// runs: from every lane a record of its own would touch 64 cache lines per
+// instruction. An odd pitch keeps the LDS banks apart. One wave per workgroup.
 template <int N>
 constexpr int kRecPitch = N | 1;
+// Elements from which they do. With fewer the chip is not full, the lines cost
+// little and the trip through LDS is latency at both ends of a wave. The fit, us
+// without / with it: 64 elements 4.0 / 9.5, 10k 5.4 / 10.5, 65k 15.3 / 16.3, and against
+// the kernel that never did 100k 27 / 20, 1M 280 / 174. The materials: 64 elements
+// 4.4 / 6.9, 300 28.8 / 28.8, against the kernel that never did 100k 101 / 66.
+constexpr int kStagedPolar = 65536, kStagedMaterial = 128;
 
-template <int N>
+template <bool STAGED, int N>
 __device__ __forceinline__ void record_in(const double* __restrict__ src, int e0, int n,
                                           double* lds, double (&v)[N]) {
   const int lane = threadIdx.x, m = min(kWave, n - e0) * N;
+  if constexpr (!STAGED) {
+    const double* p = src + (size_t)min(e0 + lane, n - 1) * N;
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = p[k];
+    return;
+  }
   __syncthreads();
   for (int i = lane; i < m; i += kWave) lds[(i / N) * kRecPitch<N> + i % N] = src[(size_t)e0 * N + i];
   __syncthreads();
@@ -1330,10 +1342,16 @@ __device__ __forceinline__ void record_in(const double* __restrict__ src, int e0
   for (int k = 0; k < N; ++k) v[k] = e0 + lane < n ? lds[lane * kRecPitch<N> + k] : 0.0;
 }
 // (half a wave's records at a time: half the LDS, twice the workgroups per CU)
-template <int N>
+template <bool STAGED, int N>
 __device__ __forceinline__ void record_out(const double (&v)[N], int e0, int n, double* lds,
                                            double* __restrict__ dst) {
   const int lane = threadIdx.x;
+  if constexpr (!STAGED) {
+    if (e0 + lane < n)
+#pragma unroll
+      for (int k = 0; k < N; ++k) dst[(size_t)(e0 + lane) * N + k] = v[k];
+    return;
+  }
 #pragma unroll 1
   for (int h = 0; h < 2; ++h) {
     const int b = e0 + h * (kWave / 2);
@@ -1347,6 +1365,7 @@ __device__ __forceinline__ void record_out(const double (&v)[N], int e0, int n, 
   }
 }
 
+template <bool STAGED>
 __global__ __launch_bounds__(kWave) void k_batch_polar(int n, const double* __restrict__ F,
                                                        double* __restrict__ R,
                                                        double* __restrict__ s,
@@ -1356,22 +1375,23 @@ __global__ __launch_bounds__(kWave) void k_batch_polar(int n, const double* __re
   static_assert(kWave * kRecPitch<9> <= kWave / 2 * kRecPitch<54>, "LDS");
   const int e0 = blockIdx.x * kWave, i = e0 + threadIdx.x;
   double Fl[9], Rl[9];
-  record_in<9>(F, e0, n, lds, Fl);
-  record_in<9>(R, e0, n, lds, Rl);
+  record_in<STAGED, 9>(F, e0, n, lds, Fl);
+  record_in<STAGED, 9>(R, e0, n, lds, Rl);
   double Sm[9], sv[6];
   int it = 0;
   if (i < n) it = procrustes_wave(Rl, Fl, 1e-6, 100);
   stretch_of(Rl, Fl, sv, Sm);
-  record_out<9>(Rl, e0, n, lds, R);
-  record_out<6>(sv, e0, n, lds, s);
+  record_out<STAGED, 9>(Rl, e0, n, lds, R);
+  record_out<STAGED, 6>(sv, e0, n, lds, s);
   if (dsdF) {
     double d[54];
     dsdF_of<double>(Rl, Fl, d);
-    record_out<54>(d, e0, n, lds, dsdF);
+    record_out<STAGED, 54>(d, e0, n, lds, dsdF);
   }
   if (iters && i < n) iters[i] = it;
 }
 
+template <bool STAGED>
 __global__ __launch_bounds__(kWave) void k_batch_material(
     int n, const int* __restrict__ type, const double* __restrict__ mu,
     const double* __restrict__ la, const double* __restrict__ s, int psd, double* __restrict__ E,
@@ -1380,18 +1400,18 @@ __global__ __launch_bounds__(kWave) void k_batch_material(
   static_assert(kWave * kRecPitch<6> <= kWave / 2 * kRecPitch<36>, "LDS");
   const int e0 = blockIdx.x * kWave, i = e0 + threadIdx.x, ic = min(i, n - 1);
   double sv[6];
-  record_in<6>(s, e0, n, lds, sv);
+  record_in<STAGED, 6>(s, e0, n, lds, sv);
   const int t = type[ic];
   if (E && i < n) E[i] = material_energy(t, mu[i], la[i], sv);
   double gg[6], HH[21];
   material_grad_hess(t, mu[ic], la[ic], sv, gg, HH);
   if (psd && i < n && material_needs_psd(t) && !chol_pd_packed<double, 6>(HH, 1e-6))
     jacobi_psd_project_packed<double, 6>(HH, 1e-6);
-  if (g) record_out<6>(gg, e0, n, lds, g);
+  if (g) record_out<STAGED, 6>(gg, e0, n, lds, g);
   if (H) {
     double A[36];
     unpack_sym6(HH, A);
-    record_out<36>(A, e0, n, lds, H);
+    record_out<STAGED, 36>(A, e0, n, lds, H);
   }
 }
 
@@ -1557,15 +1577,17 @@ void launch_mixed2d_energy(const TetMeshDev& m, const double* x_full, const doub
 void launch_batch_polar(int n, const double* F, double* R, double* s, double* dsdF, int* iters,
                         hipStream_t st) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_batch_polar, dim3(grid_for(n, 64)), dim3(64), 0, st, n, F, R, s, dsdF, iters);
+  auto kernel = n < kStagedPolar ? k_batch_polar<false> : k_batch_polar<true>;
+  hipLaunchKernelGGL(kernel, dim3(grid_for(n, 64)), dim3(64), 0, st, n, F, R, s, dsdF, iters);
 }
 
 void launch_batch_material(int n, const int* type, const double* mu, const double* la,
                            const double* s, int psd, double* E, double* g, double* H,
                            hipStream_t st) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_batch_material, dim3(grid_for(n, 64)), dim3(64), 0, st, n, type, mu, la, s,
-                     psd, E, g, H);
+  auto kernel = n < kStagedMaterial ? k_batch_material<false> : k_batch_material<true>;
+  hipLaunchKernelGGL(kernel, dim3(grid_for(n, 64)), dim3(64), 0, st, n, type, mu, la, s, psd, E, g,
+                     H);
 }
 
 void launch_batch_snh_f9(int n, const double* mu, const double* la, const double* F, double* E,

@@ -19,17 +19,30 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 31, 32, 33, 63, 64, 65])
 def test_records_at_wave_edges(n, oracle):
     from mfem_amd import native
+    check_records(native, oracle, n, range(n), range(n))
+
+
+# the lines from which records pass through LDS: 128 (material) and 65536 (fit)
+@pytest.mark.parametrize("n", [127, 128, 129, 160, 65535, 65536, 65537, 65567, 65568, 65569])
+def test_records_at_the_staging_lines(n, oracle):
+    from mfem_amd import native
+    tail = range(max(0, n - 130), n)
+    check_records(native, oracle, n, tail if n > 1000 else range(n), tail)
+
+
+def check_records(native, oracle, n, fits, materials):
     rng = np.random.RandomState(n)
     F = np.eye(3) + 0.15 * rng.uniform(-1, 1, (n, 3, 3))
     mu, la = scenes.enu_to_lame(1e6, 0.45)
     S = np.array([1, 1, 1, 0, 0, 0.0]) + 0.2 * rng.uniform(-1, 1, (n, 6))
     R, s, dsdF, it = native.polar_batch(F)
     E, g, H = native.material_s6_batch(0, mu, la, S)
-    for i in range(n):
+    for i in fits:
         Ro, so, do, _, ito = oracle.polar_svd3(F[i])
         assert it[i] == ito
         assert np.abs(R[i] - Ro).max() < 1e-12 and np.abs(s[i] - so).max() < 1e-12
         assert np.abs(dsdF[i] - do).max() < 1e-10 * np.abs(do).max()
+    for i in materials:
         Eo, go, Ho = oracle.material_s6(0, mu, la, S[i], True)
         assert abs(E[i] - Eo) <= 1e-12 * max(abs(Eo), mu)
         assert np.abs(g[i] - go).max() <= 1e-12 * max(np.abs(go).max(), mu)
