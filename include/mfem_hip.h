@@ -187,8 +187,8 @@ int mfem_sim_set_cg_shape(mfem_sim* sim, int variant, int blocks);
 /* CG kernel autotuner result: every (shape, grid) pair timed on the first
  * solve (times[count] ms per iteration, variants[count], grids[count]; pass
  * NULL arrays to query count), the index of the chosen pair (-1 when untuned
- * or forced; count is 0 where the resident kernel solves), and the chosen lanes-per-row / blocks in flight per lane /
- * workgroup size / grid. */
+ * or forced; count is 0 where the resident kernel solves), and the chosen
+ * lanes-per-row / blocks in flight per lane / workgroup size / grid. */
 int mfem_sim_cg_tuning(mfem_sim* sim, double* times, int* variants, int* grids, int* count,
                        int* chosen, int* lanes, int* unroll, int* threads, int* blocks);
 

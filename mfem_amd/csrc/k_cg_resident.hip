@@ -19,18 +19,19 @@
 //   q_it = K p; publish q_it and the workgroup's partial sums
 //
 // Measured on MI355X, us per iteration against the one-kernel-per-iteration CG:
-// 468 rows FP64 2.9 (8.1), 4840 rows FP64 3.5 (9.2), 37.5k rows FP64 5.2 (16),
-// 54.8k rows FP32 6.5 (13.2), 168k rows FP32 15 (26). What is left of a small
+// 468 rows FP64 2.9 (8.1), 4840 rows FP64 3.5 (9.2), 37.5k rows FP64 4.9 (16),
+// 54.8k rows FP32 6.3 (13.2), 168k rows FP32 14.3 (26). What is left of a small
 // system's 2.9 us is the exchange (0.6 us on one XCD, 1-2 us over all), three
 // workgroup barriers, two chains of wave sums, the two divisions and the loads
 // of q.
 //
 // Exchange. Every published word is its own flag: buffers hold a signalling
 // NaN (no arithmetic produces one) until the value is stored, and a reader
-// polls the word itself. Words are relaxed agent-scope atomics, which go past
-// the L2s that the XCDs do not share, so no cache is written back or
-// invalidated; no ordering between different words is needed except for the
-// reset below. Three slots rotate with the iteration:
+// polls the word itself. Words are relaxed agent-scope atomics, which are
+// coherent between the XCDs without any cache being written back or invalidated
+// (while one XCD alone touches a word its L2 serves it in 0.1 us; store to load
+// across XCDs takes 1-2 us); no ordering between different words is needed except
+// for the reset below. Three slots rotate with the iteration:
 //   - a workgroup publishes its sums of `it` only after all its lanes have read
 //     every word of it-1 that they need, so once all sums of it-1 have arrived,
 //     nobody reads slot it-2 any more, and its owner resets it;
@@ -673,10 +674,11 @@ bool needs_spill(int R, int max_row, int value_bytes) {
 // there are CUs left. Up to 32 workgroups stay on one XCD (every eighth
 // workgroup of the launch), whose L2 they share: 468 rows in FP64 take 2.9 us
 // an iteration on 16 workgroups of one XCD, 3.9 us on 64 over all of them; 4840
-// rows 4.5 us on the 32 of one XCD, 3.4 us on 96.
-// 31 of an XCD's 32 CUs at most: kernels of other streams still find a CU while
-// a solve spins (256 instead of 248 workgroups gained nothing: 15.0 us an
-// iteration at 168k rows either way).
+// rows 4.5 us on the 32 of one XCD, 3.5 us on three times as many over all.
+// Over all XCDs 31 CUs of each at most: kernels of other streams still find one
+// while a solve spins (256 instead of 248 workgroups gained nothing: 15.0 us an
+// iteration at 168k rows either way). A small system may take a whole XCD, a batch
+// takes every CU.
 CgResidentPlan cg_resident_plan(int nrows, int max_row, int value_bytes) {
   constexpr int kMaxWg = kCgResidentMaxWg / 32 * 31;
   CgResidentPlan P;

@@ -5,9 +5,10 @@ MI355X.
 
 Records against the oracle with the bounds of the element-level parity tests.
 Shared trials against the same elements one to a launch, where a lane has no
-helpers: both form the same trials (0.6^j w by powers against one product after
-the other, up to 100 roundings of 1e-16) and accept by one rule, so iteration
-counts are equal and R agrees to 100 applied rotations of that rounding, 1e-12."""
+helpers: both form the same trials (w shrunk by one product after the other, as the
+lane itself would) and accept by one rule, so iteration counts are equal; different
+contractions of the two loops leave R equal to 100 applied rotations of a rounding
+of 1e-16 each, 1e-12."""
 import numpy as np
 import pytest
 
