@@ -300,6 +300,8 @@ def test_solves_that_stop_at_once(native, nb):
         assert not torch.any(x != 0)
     x, it, rr = native.pcg_bsr3(rp, col, K, b, 1e-12, 10)
     assert torch.equal(x, 0.5 * b)
+    x, it, rr = native.pcg_bsr3(rp, col, K, b, 1e-12, 10, x=b)  # in place
+    assert torch.equal(x, 0.5 * torch.ones_like(b))
 
 
 @pytest.mark.parametrize("n", [(1, 1, 1), (4, 3, 2), (9, 7, 5), (20, 16, 13), (40, 40, 32)])
